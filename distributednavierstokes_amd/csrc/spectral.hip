@@ -11,6 +11,8 @@
 
 #include "closure.hpp"
 #include "host_util.hpp"
+#include "sp_x2.hpp"
+#include "sp_x2_shapes.hpp"
 #include "spectral_kernels.hpp"
 
 namespace dns {
@@ -21,6 +23,31 @@ static const double W_B[3] = {1.0 / 4.0, 0.0, 0.0};
 static const double W_DC[3] = {8.0 / 15.0, 2.0 / 15.0, 1.0 / 3.0};
 
 constexpr int SP_XEPT = 8, SP_SEPT = 8, SP_MAXO = 6, SP_NTHR = 256, SP_REDB = 1024;
+
+// The wavefront x pass (sp_x2.hpp): lines per wavefront of half length N
+// (0: not served) and its launch.  FP64 stops at N2 = 12: the registers of
+// three components of 15 or 16 points per lane spill (450-540 B per lane).
+bool sp_x2_f32_lo(const X2Args<float> &, int, int, hipStream_t);
+bool sp_x2_f32_hi(const X2Args<float> &, int, int, hipStream_t);
+bool sp_x2_f64_lo(const X2Args<double> &, int, int, hipStream_t);
+bool sp_x2_f64_hi(const X2Args<double> &, int, int, hipStream_t);
+static bool sp_x2_go(const X2Args<float> &a, int blocks, int waves, hipStream_t st)
+{
+    return sp_x2_f32_lo(a, blocks, waves, st) || sp_x2_f32_hi(a, blocks, waves, st);
+}
+static bool sp_x2_go(const X2Args<double> &a, int blocks, int waves, hipStream_t st)
+{
+    return sp_x2_f64_lo(a, blocks, waves, st) || sp_x2_f64_hi(a, blocks, waves, st);
+}
+template <typename T> static int sp_x2_lines(int N)
+{
+#define X(A, B) \
+    if (N == (A) * (B) && (sizeof(T) == 4 || (B) <= 12)) return 64 / (A);
+    SP_X2_SHAPES_LO
+    SP_X2_SHAPES_HI
+#undef X
+    return 0;
+}
 
 enum { SFAM_Y = 0, SFAM_Z = 1, SFAM_X = 2, SFAM_STAGE = 3, SFAM_FORCE = 4 };
 
@@ -64,6 +91,7 @@ template <typename T> struct SpecImpl : SpecBase {
     int tb = 1, tbf = 1, tbs = 1, lpb = 1;
     int xr_lpi = 0, xr_blocks = 0; // persistent RHS x pass: lines per block, blocks (0: k_sp_xmid)
     bool xr_wave = false;          // RHS x pass with one wavefront per line (k_sp_xrhs256, n = 512)
+    int x2_lpw = 0, x2_waves = 0, x2_blocks = 0; // wavefront x pass (k_sp_x2): lines per wavefront (0: not used), launch
     size_t ldsxr = 0;
     size_t lds = 0, ldss = 0, ldsx = 0;
     double *red = nullptr, *redout = nullptr, *factors = nullptr, *pinned = nullptr;
@@ -157,7 +185,22 @@ template <typename T> struct SpecImpl : SpecBase {
             const char *ew = getenv("DNS_SP_XWAVE");
             xr_wave = g.n == 512 && !(ew && atoi(ew) == 0);
         }
-        redcap = std::max<size_t>((size_t)SP_REDB * 4, 2 * ((size_t)g.n * g.n / lpb + 16));
+        // The wavefront x pass wherever the half length has a split (whole
+        // steps against the block kernels, forced box, MI355X: 384³ FP32
+        // 8.1 -> 5.8 ms, 384³ FP64 14.7 -> 11.0 (its 212 B of spills
+        // included), 288³ FP64 5.9 -> 4.4, 256³ FP32 2.25 -> 1.7, 64³ FP64
+        // 0.35 -> 0.32); 512-point FP64 and FP32 lines keep k_sp_xrhs256
+        // for the RHS (FP32 11.5 against 11.8 ms).  An explicit
+        // DNS_SP_XRHS keeps the block kernels.
+        if (!getenv("DNS_SP_XRHS") && g.K <= g.n / 2) x2_lpw = sp_x2_lines<T>(g.n / 2);
+        if (x2_lpw) {
+            // four wavefronts share a block's twiddles; one per block where
+            // that leaves too few blocks to spread over the CUs
+            const int waves = ceil_div((long)g.n * g.n, x2_lpw);
+            x2_waves = waves >= 8192 ? 4 : 1;
+            x2_blocks = ceil_div(waves, x2_waves);
+        }
+        redcap = std::max<size_t>({(size_t)SP_REDB * 4, 2 * ((size_t)g.n * g.n / lpb + 16), 2 * ((size_t)x2_blocks + 16)});
         DNS_TRY(dalloc(&red, redcap));
         DNS_TRY(dalloc(&redout, 64));
         DNS_TRY(dalloc(&factors, 4096));
@@ -253,8 +296,29 @@ template <typename T> struct SpecImpl : SpecBase {
 
     // vpart: per-block velocity bounds (stage 1 and vsummax read them; later
     // stages write to the scratch half of the reduction buffer)
-    template <int MODE> int xpass(double *vpart, T *physbuf = nullptr)
+    // tau: physical stress added to the products (k_sp_x2 only)
+    template <int MODE> int xpass(double *vpart, T *physbuf = nullptr, const T *tau = nullptr)
     {
+        if (x2_lpw && !(MODE == XMID_RHS && xr_wave)) {
+            X2Args<T> x;
+            x.P = P;
+            x.phys = physbuf ? physbuf : phys;
+            x.tau = tau;
+            x.vpart = vpart == red && (MODE == XMID_RHS || MODE == XMID_VMAX) ? vpart : nullptr; // scratch is not read
+            x.tw = twN;
+            x.twx = twx;
+            x.n = g.n;
+            x.K = g.K;
+            x.mode = MODE;
+            timer.begin(SFAM_X);
+            if (!sp_x2_go(x, x2_blocks, x2_waves, st)) {
+                set_error("no wavefront x pass for n = %d", g.n);
+                return DNS_EUNSUPPORTED;
+            }
+            timer.end(SFAM_X);
+            DNS_HIP_CHECK(hipGetLastError());
+            return DNS_OK;
+        }
         XMidArgs<T> a;
         a.P = P;
         a.phys = physbuf ? physbuf : phys;
@@ -397,16 +461,34 @@ template <typename T> struct SpecImpl : SpecBase {
     }
 
     // LES step with a learned sub-filter stress: each stage evaluates the
-    // network on the physical velocity, transforms τ to (K, m, m, 6) and adds
-    // it to σ̂ inside the fused stage (du_i = −ik_j(σ̂_ij + τ̂_ij)).
+    // network on the physical velocity and adds τ to the products
+    // (du_i = −ik_j(σ̂_ij + τ̂_ij)), in physical space where the wavefront x
+    // pass serves n, else as τ̂ (K, m, m, 6) inside the fused y stage.
     T *tphys = nullptr; // physical τ (n³ × 6)
     int closure_step(dns_cnn *net, double dt, double *vmax)
     {
         DNS_TRY(ensure_phys());
-        DNS_TRY(ensure_aux());
-        if (!du) DNS_TRY(dalloc(&du, 3 * ns));
         const size_t n3 = (size_t)g.n * g.n * g.n;
         if (!tphys) DNS_TRY(dalloc(&tphys, 6 * n3));
+        if (x2_lpw && !xr_wave) {
+            // the stress joins the products in physical space (the transform
+            // is linear), and the velocity pencils in P outlive the c2r into
+            // phys, so a stage runs no second backward transform and no
+            // transform of τ of its own: 6 launches beside the network's
+            // instead of 14
+            for (int s = 0; s < 3; ++s) {
+                DNS_TRY(backward_yz());
+                DNS_TRY(xpass<XMID_C2R>(nullptr));
+                DNS_TRY(cnn_stress<T>(net, phys, tphys, g.n, st));
+                DNS_TRY(xpass<XMID_RHS>(s == 0 ? red : nullptr, nullptr, tphys));
+                DNS_TRY(zfwd(6));
+                DNS_TRY(ystage<0>(s, dt));
+            }
+            if (vmax) DNS_TRY(vmax_final(rhs_parts(), vmax));
+            return DNS_OK;
+        }
+        DNS_TRY(ensure_aux());
+        if (!du) DNS_TRY(dalloc(&du, 3 * ns));
         for (int s = 0; s < 3; ++s) {
             DNS_TRY(backward_yz());
             DNS_TRY(xpass<XMID_C2R>(red + redcap / 2));
@@ -461,6 +543,7 @@ template <typename T> struct SpecImpl : SpecBase {
     int rhs_parts() const
     {
         if (xr_wave) return (int)ceil_div((long)g.n * g.n, 4);
+        if (x2_lpw) return x2_blocks;
         return xr_lpi ? xr_blocks : (int)ceil_div((long)g.n * g.n, lpb);
     }
 
@@ -495,7 +578,7 @@ template <typename T> struct SpecImpl : SpecBase {
     {
         DNS_TRY(backward_yz());
         DNS_TRY(xpass<XMID_VMAX>(red));
-        return vmax_final(ceil_div((long)g.n * g.n, lpb), out);
+        return vmax_final(x2_lpw ? x2_blocks : ceil_div((long)g.n * g.n, lpb), out);
     }
 
     long cube_count(int r) const

@@ -1,0 +1,46 @@
+"""Wavefront x pass of the spectral step (k_sp_x2): one case per shape at the
+edges of its range, against the oracle's transforms and step."""
+import numpy as np
+import pytest
+
+import distributednavierstokes_amd as dns
+from distributednavierstokes_amd.problem import SpectralProblem
+from oracle.oracle import OracleSpectral
+
+pytestmark = pytest.mark.gpu
+
+# smallest and largest half lengths, every radix of the small DFTs (2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16), odd and
+# prime-power half lengths, line counts that leave partly filled wavefronts
+SIZES = [32, 36, 40, 50, 54, 64, 72, 96, 120, 150, 160]
+
+
+def cases():
+    for n in SIZES:
+        yield n, n // 3, np.float64
+        yield n, n // 3, np.float32
+    yield 48, 5, np.float64  # few retained modes: whole register rows beyond K
+    yield 48, 5, np.float32
+
+
+@pytest.mark.parametrize("n,kcut,T", list(cases()))
+def test_x2_transforms_and_step(n, kcut, T):
+    """spec_to_phys, phys_to_spec, max Σ|v| and one RHS step.  Bounds: an FFT
+    pass of N points rounds by a few eps log2 N relative to the field's
+    maximum; 1e-12 and 2e-5 are the bounds of the other transform tests."""
+    tol = 1e-12 if T == np.float64 else 2e-5
+    s = dns.spectral_setup(n=n, visc=5e-3, kcut=kcut, T=T)
+    o = OracleSpectral(SpectralProblem(n=n, visc=5e-3, kcut=kcut))
+    uh = o.randomfield(totalenergy=0.5, kpeak=3, seed=n)
+    v = o.spec_to_phys(uh)
+    vg = np.zeros_like(v, order="F")
+    dns.spec_to_phys_(vg, uh, s)
+    assert np.abs(vg - v).max() <= tol * np.abs(v).max()
+    w = o.phys_to_spec(v)
+    wg = np.zeros_like(uh)
+    dns.phys_to_spec_(wg, v, s)
+    assert np.abs(wg - w).max() <= tol * np.abs(w).max()
+    ref, got = uh.copy(order="F"), uh.copy(order="F")
+    vr = o.step(ref, 1e-3)
+    vm = dns.spectral_step_(got, s, 1e-3)
+    assert abs(vm - vr) <= tol * vr
+    assert np.abs(got - ref).max() <= tol * np.abs(ref).max()
