@@ -1,6 +1,7 @@
 // Small DFTs in registers for the two-step line transforms: radices that are
-// products of the primitive ones of fft_lds.hpp (6, 9, 10, 12, 15, 16), with
-// their inner twiddles folded to constants.
+// products of the primitive ones of fft_lds.hpp (6, 9, 10, 12, 15, 16, 18, 20,
+// 24, 25, 27, 32), with their inner twiddles folded to
+// constants.
 #pragma once
 
 #include "fft_lds.hpp"
@@ -96,5 +97,11 @@ template <typename T, bool INV> struct Dft<T, 10, INV> : DftC<T, 2, 5, INV> {};
 template <typename T, bool INV> struct Dft<T, 12, INV> : DftC<T, 4, 3, INV> {};
 template <typename T, bool INV> struct Dft<T, 15, INV> : DftC<T, 5, 3, INV> {};
 template <typename T, bool INV> struct Dft<T, 16, INV> : DftC<T, 4, 4, INV> {};
+template <typename T, bool INV> struct Dft<T, 18, INV> : DftC<T, 6, 3, INV> {};
+template <typename T, bool INV> struct Dft<T, 20, INV> : DftC<T, 4, 5, INV> {};
+template <typename T, bool INV> struct Dft<T, 24, INV> : DftC<T, 8, 3, INV> {};
+template <typename T, bool INV> struct Dft<T, 25, INV> : DftC<T, 5, 5, INV> {};
+template <typename T, bool INV> struct Dft<T, 27, INV> : DftC<T, 9, 3, INV> {};
+template <typename T, bool INV> struct Dft<T, 32, INV> : DftC<T, 8, 4, INV> {};
 
 }  // namespace dns

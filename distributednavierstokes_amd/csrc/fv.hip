@@ -12,6 +12,7 @@
 #include "fv_kernels.hpp"
 #include "plain_kernels.hpp"
 #include "host_util.hpp"
+#include "p2.hpp"
 
 namespace dns {
 
@@ -513,6 +514,14 @@ template <typename T> struct FVImpl : FVBase {
                 }
             }
         }
+        // two-step pencil passes (32-bit byte offsets within the pencil array);
+        // measured against the LDS tiles, ms per explicit step: 64³ 0.17 ->
+        // 0.14, 96x90x60 0.27 -> 0.20, 256³ 2.71 -> 2.64, 256³ mixed 1.56 ->
+        // 1.41, 512x384x512 CN unchanged (its z pass was at the copy rate)
+        if ((size_t)g.ldc * ny * nz * sizeof(cplx<T>) < ((size_t)1 << 31)) {
+            p2_z = p2_serves<T>(P2_FULL, nz);
+            p2_y = !g.wall && p2_serves<T>(P2_FOURIER, ny);
+        }
         if (ldsz > (size_t)maxlds || ldsy > (size_t)maxlds) {
             set_error("FFT tile does not fit the %d-byte LDS limit", maxlds);
             return DNS_EUNSUPPORTED;
@@ -713,12 +722,56 @@ template <typename T> struct FVImpl : FVBase {
         return DNS_OK;
     }
 
+    // two-step pencil passes (p2.hpp) of lines of n points, `stride` apart, one
+    // row of kx lines every `row` elements; 128-byte rows per block
+    bool p2_z = false, p2_y = false;
+    P2Args<T> p2_lines(cplx<T> *A_, const cplx<T> *tw, int n, size_t stride, size_t row) const
+    {
+        P2Args<T> a{};
+        a.dst = A_;
+        a.dst1 = row;
+        a.dstride = (int)stride;
+        a.tw = tw;
+        a.n = n;
+        a.K = g.nxc;
+        a.lb = sizeof(T) == 8 ? 3 : 4;
+        a.scale = T(1);
+        return a;
+    }
+
+    // the periodic y pass of A_: forward, divided by the eigenvalues (times
+    // scale) and back, or (divide = false) forward only
+    void launch_fourier_y(cplx<T> *A_, bool divide, double scale)
+    {
+        if (p2_y) {
+            P2Args<T> a = p2_lines(A_, twy, g.ny, g.ldc, (size_t)g.ldc * g.ny);
+            a.lam1 = lam1;
+            a.lam2 = lam2;
+            a.lam3 = lam3;
+            a.dscale = scale;
+            p2_launch(divide ? P2_FOURIER : P2_FULL, a, dim3(ceil_div(g.nxc, 1 << a.lb), g.nz), st);
+            return;
+        }
+        const dim3 grd(ceil_div(g.nxc, tby), g.nz);
+        if (divide)
+            hipLaunchKernelGGL((k_fourier_y<T, ZY_EPT, true>), grd, dim3(nthry), ldsy, st, A_, twy, lam1, lam2, lam3,
+                               scale, tby, tbyf, make_fastdiv(tby), g, fdy);
+        else
+            hipLaunchKernelGGL((k_fourier_y<T, ZY_EPT, false>), grd, dim3(nthry), ldsy, st, A_, twy, lam1, lam2, lam3,
+                               scale, tby, tbyf, make_fastdiv(tby), g, fdy);
+    }
+
     // poisson! of the divergence of uu, writing the pressure into psi
     // (src/poisson.jl:147-161), without transposes: x pass, z pass, y solve,
     // in-place z FFT of the (nxc, ny, nz) pencil A (k_fft_z, 256- or
     // 512-thread tiles)
     template <bool INV> void launch_fft_z(cplx<T> *A_)
     {
+        if (p2_z) {
+            P2Args<T> a = p2_lines(A_, twz, g.nz, (size_t)g.ldc * g.ny, g.ldc);
+            p2_launch(INV ? P2_FULLI : P2_FULL, a, dim3(ceil_div(g.nxc, 1 << a.lb), g.ny), st);
+            return;
+        }
         const dim3 grd(ceil_div(g.nxc, tbz), g.ny);
         if (nthrz == 2 * NTHR)
             hipLaunchKernelGGL((k_fft_z<T, ZY_EPT, INV, 2 * NTHR>), grd, dim3(nthrz), ldsz, st, A_, twz, tbz, tbzf,
@@ -803,8 +856,7 @@ template <typename T> struct FVImpl : FVBase {
             }
         } else {
             double scale = 1.0 / ((double)g.nx * g.ny * g.nz);
-            hipLaunchKernelGGL((k_fourier_y<T, ZY_EPT, true>), dim3(ceil_div(g.nxc, tby), g.nz), dim3(nthry), ldsy,
-                               st, A, twy, lam1, lam2, lam3, scale, tby, tbyf, make_fastdiv(tby), g, fdy);
+            launch_fourier_y(A, true, scale);
         }
         timer.end(FAM_Y);
         DNS_HIP_CHECK(hipGetLastError());
@@ -1075,8 +1127,7 @@ template <typename T> struct FVImpl : FVBase {
             hipLaunchKernelGGL((k_thomas_y<T>), dim3(ceil_div(lines, NTHR)), dim3(NTHR), 0, st, pC, Dth, iptab, ay, cy,
                                lam1, lam3, 1.0 / ((double)g.nx * g.nz), g);
         } else {
-            hipLaunchKernelGGL((k_fourier_y<T, ZY_EPT, true>), dim3(ceil_div(g.nxc, tby), g.nz), dim3(nthry), ldsy,
-                               st, pC, twy, lam1, lam2, lam3, 1.0 / ((double)g.nx * g.ny * g.nz), tby, tbyf, make_fastdiv(tby), g, fdy);
+            launch_fourier_y(pC, true, 1.0 / ((double)g.nx * g.ny * g.nz));
         }
         timer.end(FAM_Y);
         timer.begin(FAM_Z);
@@ -1186,8 +1237,11 @@ template <typename T> struct FVImpl : FVBase {
         char xdesc[32];
         if (xwave) snprintf(xdesc, sizeof xdesc, "wave groups of %d", g.nx / 8);
         else snprintf(xdesc, sizeof xdesc, "lpb=%d", lpb);
-        char ys[64], cs[96];
-        if (!g.wall) snprintf(ys, sizeof ys, "fourier n=%d tile=%d/%d thr=%d", g.ny, tby, tbyf, nthry);
+        char ys[64], cs[96], zs[64];
+        if (p2_z) snprintf(zs, sizeof zs, "n %d two-step", g.nz);
+        else snprintf(zs, sizeof zs, "n %d tile=%d/%d thr=%d", g.nz, tbz, tbzf, nthrz);
+        if (p2_y) snprintf(ys, sizeof ys, "fourier n=%d two-step", g.ny);
+        else if (!g.wall) snprintf(ys, sizeof ys, "fourier n=%d tile=%d/%d thr=%d", g.ny, tby, tbyf, nthry);
         else if (thomas_tl && thomas_seg) snprintf(ys, sizeof ys, "seg R=%d tl=%d thr=%d", thomas_seg, thomas_tl, thomas_nthr);
         else if (thomas_tl) snprintf(ys, sizeof ys, "tile tl=%d thr=%d", thomas_tl, thomas_nthr);
         else snprintf(ys, sizeof ys, "sequential");
@@ -1197,10 +1251,10 @@ template <typename T> struct FVImpl : FVBase {
         else if (cn_tl) snprintf(cs, sizeof cs, "tile tl=%d thr=%d", cn_tl, cn_nthr);
         else snprintf(cs, sizeof cs, "sequential");
         const int n = snprintf(buf, (size_t)len,
-                               "prec=%s; momentum=%s zc=%d; xpass=half %d %s; zpass=n %d tile=%d/%d thr=%d; "
+                               "prec=%s; momentum=%s zc=%d; xpass=half %d %s; zpass=%s; "
                                "ysolve=%s; cn=%s; pgrad=%s",
                                plain ? "plain" : sizeof(T) == 8 ? "fp64" : "mixed", mom, momentum_zc(), g.nx / 2, xdesc,
-                               g.nz, tbz, tbzf, nthrz, ys, cs, pgrad_vec ? "vec" : "scalar");
+                               zs, ys, cs, pgrad_vec ? "vec" : "scalar");
         if (n < 0 || n >= len) {
             set_error("describe: buffer of %d bytes too small", len);
             return DNS_EINVAL;
@@ -1605,8 +1659,7 @@ template <typename T> struct FVImpl : FVBase {
             hipLaunchKernelGGL((k_rfft_x<T, X_EPT, 1>), dim3(ceil_div(g.ny * g.nz, lpb)), dim3(NTHR), ldsx, st, xa, g,
                                fdx);
             launch_fft_z<false>(A);
-            hipLaunchKernelGGL((k_fourier_y<T, ZY_EPT, false>), dim3(ceil_div(g.nxc, tby), g.nz), dim3(nthry), ldsy,
-                               st, A, twy, lam1, lam2, lam3, 1.0, tby, tbyf, make_fastdiv(tby), g, fdy);
+            launch_fourier_y(A, false, 1.0);
             if (nbins <= 2048)
                 hipLaunchKernelGGL((k_binshells_w<T>), dim3(nb), dim3(NTHR), sizeof(double) * 4 * nbins, st, A, g,
                                    nbins, 1.0 / N2, spart);

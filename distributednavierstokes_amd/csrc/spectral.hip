@@ -11,6 +11,7 @@
 
 #include "closure.hpp"
 #include "host_util.hpp"
+#include "p2.hpp"
 #include "sp_x2.hpp"
 #include "sp_x2_shapes.hpp"
 #include "spectral_kernels.hpp"
@@ -200,6 +201,16 @@ template <typename T> struct SpecImpl : SpecBase {
             x2_waves = waves >= 8192 ? 4 : 1;
             x2_blocks = ceil_div(waves, x2_waves);
         }
+        // two-step pencil passes (32-bit byte offsets within a line's span)
+        if ((size_t)g.K * g.n * g.n * sizeof(cplx<T>) < ((size_t)1 << 31)) {
+            // 128-byte rows; measured against the LDS tiles on the forced box,
+            // ms per step: 96³ FP64 0.45 -> 0.31, 192³ FP64 1.49 -> 1.32, 512³
+            // FP64 21.6 -> 20.3; 96³ FP32 0.41 -> 0.26, 384³ FP32 5.88 -> 5.16,
+            // 512³ FP32 11.7 -> 11.0 (64-byte rows 12-15 % slower there)
+            p2_pencil = p2_serves<T>(P2_FWD, g.n);
+            p2_stage = p2_serves<T>(P2_STAGE, g.n);
+            p2_lb = sizeof(T) == 8 ? 3 : 4;
+        }
         redcap = std::max<size_t>({(size_t)SP_REDB * 4, 2 * ((size_t)g.n * g.n / lpb + 16), 2 * ((size_t)x2_blocks + 16)});
         DNS_TRY(dalloc(&red, redcap));
         DNS_TRY(dalloc(&redout, 64));
@@ -215,6 +226,48 @@ template <typename T> struct SpecImpl : SpecBase {
         out->l = l;
         out->visc = visc;
         out->precision = sizeof(T) == 8 ? DNS_FP64 : DNS_MIXED;
+    }
+
+    // ------------------------------------------- two-step pencil passes
+    bool p2_pencil = false, p2_stage = false; // p2.hpp instead of the LDS tiles (y/z passes; IF-stage pass)
+    int p2_lb = 0;                            // log2 of their lines per block
+
+    P2Args<T> p2_args() const
+    {
+        P2Args<T> a{};
+        a.tw = twn;
+        a.n = g.n;
+        a.K = g.K;
+        a.lb = p2_lb;
+        a.kcut = g.kcut;
+        a.m = g.m;
+        a.scale = T(1);
+        return a;
+    }
+
+    // lines along y (stride K, fixed kz = block row) or z (stride K n, fixed
+    // y) of nc components; pn: planes per component on each side
+    int p2_pass(P2Kind kind, const cplx<T> *src, cplx<T> *dst, bool alongz, int nc, T scale)
+    {
+        P2Args<T> a = p2_args();
+        const size_t K = g.K, n = g.n, m = g.m;
+        const size_t fine = alongz ? K : K * n, comp = alongz ? K : K * m; // block-row steps of full and compact lines
+        const bool back = kind == P2_BACK;
+        a.src = src;
+        a.dst = dst;
+        a.scale = scale;
+        a.sstride = a.dstride = (int)(alongz ? K * n : K);
+        a.src1 = back ? comp : fine;
+        a.dst1 = back ? fine : comp;
+        const size_t sc = alongz ? K * n * m : K * m * m, sf = alongz ? K * n * n : K * n * m;
+        a.src2 = back ? sc : sf;
+        a.dst2 = back ? sf : sc;
+        const dim3 grd(ceil_div(g.K, 1 << a.lb), alongz ? g.n : g.m, nc);
+        if (!p2_launch(kind, a, grd, st)) {
+            set_error("no two-step pencil pass for n = %d", g.n);
+            return DNS_EUNSUPPORTED;
+        }
+        return DNS_OK;
     }
 
     // --------------------------------------------------------- transfers
@@ -282,6 +335,16 @@ template <typename T> struct SpecImpl : SpecBase {
     // ----------------------------------------------------------- passes
     int backward_yz(const cplx<T> *src = nullptr)
     {
+        if (p2_pencil) {
+            timer.begin(SFAM_Y);
+            DNS_TRY(p2_pass(P2_BACK, src ? src : uh, Q, false, 3, T(1)));
+            timer.end(SFAM_Y);
+            timer.begin(SFAM_Z);
+            DNS_TRY(p2_pass(P2_BACK, Q, P, true, 3, T(1)));
+            timer.end(SFAM_Z);
+            DNS_HIP_CHECK(hipGetLastError());
+            return DNS_OK;
+        }
         timer.begin(SFAM_Y);
         hipLaunchKernelGGL((k_sp_yback<T, SP_EPT, SP_NTHR>), dim3(ceil_div(g.K, tb), g.m, 3), dim3(SP_NTHR), lds, st,
                            src ? src : uh, Q, twn, tb, tbf, make_fastdiv(tb), g, fdn);
@@ -347,6 +410,12 @@ template <typename T> struct SpecImpl : SpecBase {
     int zfwd(int ncomp)
     {
         timer.begin(SFAM_Z);
+        if (p2_pencil) {
+            DNS_TRY(p2_pass(P2_FWD, P, Q, true, ncomp, T(1)));
+            timer.end(SFAM_Z);
+            DNS_HIP_CHECK(hipGetLastError());
+            return DNS_OK;
+        }
         hipLaunchKernelGGL((k_sp_zfwd<T, SP_EPT, SP_NTHR>), dim3(ceil_div(g.K, tb), g.n, ncomp), dim3(SP_NTHR), lds, st, P, Q,
                            twn, tb, tbf, make_fastdiv(tb), g, fdn);
         timer.end(SFAM_Z);
@@ -354,8 +423,44 @@ template <typename T> struct SpecImpl : SpecBase {
         return DNS_OK;
     }
 
+    // forward y pass of nc components of Q into compact spectra, times 1/n³
+    int yfwd(cplx<T> *dst, int nc)
+    {
+        if (p2_pencil) {
+            DNS_TRY(p2_pass(P2_FWD, Q, dst, false, nc, T(1.0 / ((double)g.n * g.n * g.n))));
+        } else {
+            hipLaunchKernelGGL((k_sp_yfwd<T, SP_EPT, SP_NTHR>), dim3(ceil_div(g.K, tb), g.m, nc), dim3(SP_NTHR), lds, st, Q,
+                               dst, twn, tb, tbf, make_fastdiv(tb), g, fdn);
+        }
+        DNS_HIP_CHECK(hipGetLastError());
+        return DNS_OK;
+    }
+
     template <int MODE> int ystage(int stage, double dt, const cplx<T> *extra = nullptr)
     {
+        if (p2_stage && !extra) {
+            P2Args<T> a = p2_args();
+            a.src = Q;
+            a.scale = T(1.0 / ((double)g.n * g.n * g.n));
+            a.uh = uh;
+            a.ustart = ustart;
+            a.du = du;
+            a.mode = MODE;
+            a.first = stage == 0;
+            a.kfac = g.kfac;
+            a.a = (T)W_A[stage];
+            a.b = (T)W_B[stage];
+            a.nudcdt = (T)(visc * W_DC[stage] * dt);
+            a.dt = (T)dt;
+            timer.begin(SFAM_STAGE);
+            if (!p2_launch(P2_STAGE, a, dim3(ceil_div(g.K, 1 << a.lb), g.m), st)) {
+                set_error("no two-step stage pass for n = %d", g.n);
+                return DNS_EUNSUPPORTED;
+            }
+            timer.end(SFAM_STAGE);
+            DNS_HIP_CHECK(hipGetLastError());
+            return DNS_OK;
+        }
         StageArgs<T> s;
         s.Q = Q;
         s.uh = uh;
@@ -400,6 +505,7 @@ template <typename T> struct SpecImpl : SpecBase {
         DNS_TRY(backward_yz());
         DNS_TRY(xpass<XMID_RHS>(red + redcap / 2));
         DNS_TRY(zfwd(6));
+        if (p2_pencil) return yfwd(P, 6);
         StageArgs<T> sa;
         sa.Q = Q;
         sa.uh = uh;
@@ -442,10 +548,7 @@ template <typename T> struct SpecImpl : SpecBase {
         DNS_TRY(ensure_phys());
         DNS_TRY(xpass<XMID_R2C>(red));
         DNS_TRY(zfwd(3));
-        hipLaunchKernelGGL((k_sp_yfwd<T, SP_EPT, SP_NTHR>), dim3(ceil_div(g.K, tb), g.m, 3), dim3(SP_NTHR), lds, st, Q, uh, twn,
-                           tb, tbf, make_fastdiv(tb), g, fdn);
-        DNS_HIP_CHECK(hipGetLastError());
-        return DNS_OK;
+        return yfwd(uh, 3);
     }
 
     // Forward transform of three physical components at src (n³ planar each)
@@ -454,10 +557,7 @@ template <typename T> struct SpecImpl : SpecBase {
     {
         DNS_TRY(xpass<XMID_R2C>(red, src));
         DNS_TRY(zfwd(3));
-        hipLaunchKernelGGL((k_sp_yfwd<T, SP_EPT, SP_NTHR>), dim3(ceil_div(g.K, tb), g.m, 3), dim3(SP_NTHR), lds, st, Q, dst, twn,
-                           tb, tbf, make_fastdiv(tb), g, fdn);
-        DNS_HIP_CHECK(hipGetLastError());
-        return DNS_OK;
+        return yfwd(dst, 3);
     }
 
     // LES step with a learned sub-filter stress: each stage evaluates the
