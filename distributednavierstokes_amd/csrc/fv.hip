@@ -517,8 +517,12 @@ template <typename T> struct FVImpl : FVBase {
         // two-step pencil passes (32-bit byte offsets within the pencil array);
         // measured against the LDS tiles, ms per explicit step: 64³ 0.17 ->
         // 0.14, 96x90x60 0.27 -> 0.20, 256³ 2.71 -> 2.64, 256³ mixed 1.56 ->
-        // 1.41, 512x384x512 CN unchanged (its z pass was at the copy rate)
-        if ((size_t)g.ldc * ny * nz * sizeof(cplx<T>) < ((size_t)1 << 31)) {
+        // 1.41, 512x384x512 CN unchanged (its z pass was at the copy rate).
+        // FP32 channels keep the tiles: their pressure is only as good as
+        // the rounding of u over Δt, and another order of rounding moved it by
+        // up to 3 % of itself where Δt is smallest (36x357x50), for 0-9 % of
+        // the step.
+        if ((size_t)g.ldc * ny * nz * sizeof(cplx<T>) < ((size_t)1 << 31) && (sizeof(T) == 8 || !g.wall)) {
             p2_z = p2_serves<T>(P2_FULL, nz);
             p2_y = !g.wall && p2_serves<T>(P2_FOURIER, ny);
         }
