@@ -23,34 +23,56 @@ struct CNNLayer {
     unsigned short *W = nullptr, *WT = nullptr;
 };
 
-// Planar (c, Vs) → channels-last BF16 with scale (one sample into one batch slot).
-template <typename T>
-__global__ void k_planar_to_bf16(const T *x, int cin, long Vs, float scale, unsigned short *out, int ldc)
+// One voxel of a planar (3, Vs) velocity → 16 BF16 channels (three of them
+// scale · u, the padding zero): two 16-byte stores.
+template <typename T> __device__ inline void velocity_to_bf16(const T *x, long Vs, long v, float scale, unsigned short *out)
 {
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < Vs * ldc; e += (long)gridDim.x * blockDim.x) {
-        const long v = e / ldc;
-        const int c = (int)(e - v * ldc);
-        out[e] = c < cin ? f2bf(scale * (float)x[(size_t)c * Vs + v]) : (unsigned short)0;
-    }
+    const unsigned short c0 = f2bf(scale * (float)x[v]), c1 = f2bf(scale * (float)x[Vs + v]),
+                         c2 = f2bf(scale * (float)x[2 * Vs + v]);
+    u32x4 *dst = reinterpret_cast<u32x4 *>(out + 16 * v);
+    dst[0] = u32x4{(unsigned)c0 | ((unsigned)c1 << 16), c2, 0u, 0u};
+    dst[1] = u32x4{0u, 0u, 0u, 0u};
 }
 
-// Planar (c, Vs) FP32 → interleaved (Vs, c) FP32 with scale.
-__global__ void k_planar_to_interleaved(const float *x, int c_, long Vs, float scale, float *out)
+// Planar (3, Vs) → 16-channel BF16 with scale, a thread per voxel (one
+// sample).  A thread per channel with a division each and 2-byte stores took
+// 18-22 µs for 64³, this 3-4.
+template <typename T> __global__ void __launch_bounds__(256) k_velocity_to_bf16(const T *x, long Vs, float scale, unsigned short *out)
 {
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < Vs * c_; e += (long)gridDim.x * blockDim.x) {
-        const long v = e / c_;
-        const int c = (int)(e - v * c_);
-        out[e] = scale * x[(size_t)c * Vs + v];
-    }
+    const long v = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (v < Vs) velocity_to_bf16<T>(x, Vs, v, scale, out);
 }
 
-// Interleaved (Vs, c) FP32 → planar (c, Vs) of T with scale.
-template <typename T> __global__ void k_interleaved_to_planar(const float *y, int c_, long Vs, double scale, T *out)
+// Dataset samples into consecutive batch slots: ū → BF16 network input, τ →
+// interleaved FP32 (Vs, 6) target, both scaled.  One launch for up to 32
+// slots (blockIdx.y) instead of two per slot.
+constexpr int STAGE_SLOTS = 32;
+struct StagePairs {
+    const float *u[STAGE_SLOTS], *t[STAGE_SLOTS];
+};
+__global__ void __launch_bounds__(256) k_stage_pairs(StagePairs p, long Vs, float su, float st, unsigned short *x0, float *t)
 {
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < Vs * c_; e += (long)gridDim.x * blockDim.x) {
-        const int c = (int)(e / Vs);
-        const long v = e - (long)c * Vs;
-        out[e] = (T)(scale * (double)y[v * c_ + c]);
+    const long v = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (v >= Vs) return;
+    const int b = blockIdx.y;
+    velocity_to_bf16<float>(p.u[b], Vs, v, su, x0 + (size_t)b * Vs * 16);
+    const float *src = p.t[b];
+    float2 *dst = reinterpret_cast<float2 *>(t + ((size_t)b * Vs + v) * 6);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) dst[c] = make_float2(st * src[2 * c * Vs + v], st * src[(2 * c + 1) * Vs + v]);
+}
+
+// Interleaved (Vs, 6) FP32 → planar (6, Vs) of T with scale, a thread per voxel.
+template <typename T> __global__ void __launch_bounds__(256) k_stress_to_planar(const float *y, long Vs, double scale, T *out)
+{
+    const long v = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (v >= Vs) return;
+    const float2 *src = reinterpret_cast<const float2 *>(y + v * 6);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const float2 p = src[c];
+        out[(size_t)(2 * c) * Vs + v] = (T)(scale * (double)p.x);
+        out[(size_t)(2 * c + 1) * Vs + v] = (T)(scale * (double)p.y);
     }
 }
 
@@ -140,6 +162,11 @@ struct CNN {
         DNS_HIP_CHECK(hipEventCreateWithFlags(&ev_in, hipEventDisableTiming));
         DNS_HIP_CHECK(hipEventCreateWithFlags(&ev_out, hipEventDisableTiming));
         timer.st = st;
+        {
+            int dev = 0, v = 0;
+            hipGetDevice(&dev);
+            if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > 0) max_lds = v;
+        }
         const char *env = getenv("DNS_CNN_MFMA");
         mfma_k8 = env && !strcmp(env, "k8");
         const char *envc = getenv("DNS_CNN_CONV");
@@ -195,7 +222,7 @@ struct CNN {
         row_wgrad = !mfma_k8 && M % 16 == 0 && M <= 256;
         const char *envw = getenv("DNS_CNN_WGRAD");
         rows_wgrad = row_wgrad && M <= 64 && envw && !strcmp(envw, "rows");
-        planes_wgrad = row_wgrad && M <= 64 && !(envw && (!strcmp(envw, "rows") || !strcmp(envw, "row16")));
+        tr_wgrad = row_wgrad && M <= 64 && !(envw && (!strcmp(envw, "rows") || !strcmp(envw, "row16")));
         if (const char *es = getenv("DNS_CNN_WSPLIT")) wgrad_splits = std::max(1, std::min(256, atoi(es)));
         const int nsplit16 = row_wgrad ? (int)std::min<long>(256, (long)B * M * M) : 0;
         DNS_TRY(dalloc(&wpart, (size_t)std::max(nsplit, nsplit16) * 27 * 64 * 64));
@@ -224,11 +251,26 @@ struct CNN {
     bool mfma_k8 = false;
     bool row_wgrad = false; // k_conv_wgrad16 (M % 16 == 0) instead of k_conv_wgrad
     bool rows_wgrad = false;   // k_conv_wgrad_rows (M % 16 == 0, M <= 64); DNS_CNN_WGRAD=rows
-    bool planes_wgrad = false; // k_conv_wgrad_planes (M % 16 == 0, M <= 64), the default
-    int wgrad_splits = 128;    // plane splits of k_conv_wgrad_planes (DNS_CNN_WSPLIT, sweep)
+    bool tr_wgrad = false;     // k_conv_wgrad_tr (M % 16 == 0, M <= 64), the default
+    // row splits of k_conv_wgrad_tr: × 3 dz, the blocks of one round at two per
+    // CU (DNS_CNN_WSPLIT, sweep)
+    int wgrad_splits = 170;
     bool row_conv = false;  // k_conv_rows (M = 32 or 64) instead of k_conv16; DNS_CNN_CONV=direct disables
-    bool conv_pf = false;   // k_conv_rows_pf at M = 64 (kin 16 or 64); DNS_CNN_CONV=rows selects k_conv_rows
-    bool conv_wlds = true;  // its weights shared through LDS; DNS_CNN_WLDS=0 streams them per wavefront
+    bool conv_pf = false;   // k_conv_plane (k_conv_rows_pf with DNS_CNN_WLDS=0); DNS_CNN_CONV=rows selects k_conv_rows
+    bool conv_wlds = true;  // weights shared through LDS; DNS_CNN_WLDS=0 streams them per wavefront (M = 64)
+    size_t max_lds = 65536;
+    template <int MC, int EPI> void conv_plane(const ConvArgs &ca, int np, long Vn, hipStream_t s)
+    {
+        const dim3 grd((unsigned)ceil_div((long)M * M, 256), (unsigned)M, (unsigned)(Vn / Vs)), blk(256);
+        const size_t lds = conv_plane_lds(M, np, ca.kin);
+        if (ca.kin == 64) {
+            if (np == 64) hipLaunchKernelGGL((k_conv_plane<MC, 2, 64, EPI>), grd, blk, lds, s, ca, geom(Vn));
+            else hipLaunchKernelGGL((k_conv_plane<MC, 1, 64, EPI>), grd, blk, lds, s, ca, geom(Vn));
+        } else {
+            if (np == 64) hipLaunchKernelGGL((k_conv_plane<MC, 2, 16, EPI>), grd, blk, lds, s, ca, geom(Vn));
+            else hipLaunchKernelGGL((k_conv_plane<MC, 1, 16, EPI>), grd, blk, lds, s, ca, geom(Vn));
+        }
+    }
     template <int EPI> void conv(const ConvArgs &ca, int np, long Vn, hipStream_t s)
     {
         if (mfma_k8) {
@@ -241,19 +283,21 @@ struct CNN {
             }
             return;
         }
+        // The plane kernel wherever its rows fit the LDS (M up to 176 or so);
+        // measured against k_conv_rows (M = 32) and k_conv16 (other M), ms per
+        // training step: see conv_plane in the table of DNS_CNN_CONV below.
+        if (conv_pf && conv_wlds && (ca.kin == 16 || ca.kin == 64) && (np == 32 || np == 64) &&
+            conv_plane_lds(M, np, ca.kin) <= max_lds) {
+            if (M == 64) conv_plane<64, EPI>(ca, np, Vn, s);
+            else if (M == 32) conv_plane<32, EPI>(ca, np, Vn, s);
+            else if (M == 16) conv_plane<16, EPI>(ca, np, Vn, s);
+            else conv_plane<0, EPI>(ca, np, Vn, s);
+            return;
+        }
         if (row_conv && (M == 32 || M == 64) && ca.kin % 16 == 0 && (np == 32 || np == 64)) {
             const dim3 grd((unsigned)(M / 4), (unsigned)M, (unsigned)(Vn / Vs));
             const size_t lds = sizeof(unsigned short) * 6 * (size_t)M * (ca.kin + 8);
-            if (conv_pf && M == 64 && (ca.kin == 16 || ca.kin == 64) && conv_wlds) {
-                const size_t ldsw = lds + sizeof(unsigned short) * 2 * (size_t)np * (ca.kin + 8);
-                if (ca.kin == 64) {
-                    if (np == 64) hipLaunchKernelGGL((k_conv_rows_pf<2, 2, 64, EPI, true>), grd, dim3(256), ldsw, s, ca, geom(Vn));
-                    else hipLaunchKernelGGL((k_conv_rows_pf<2, 1, 64, EPI, true>), grd, dim3(256), ldsw, s, ca, geom(Vn));
-                } else {
-                    if (np == 64) hipLaunchKernelGGL((k_conv_rows_pf<2, 2, 16, EPI, true>), grd, dim3(256), ldsw, s, ca, geom(Vn));
-                    else hipLaunchKernelGGL((k_conv_rows_pf<2, 1, 16, EPI, true>), grd, dim3(256), ldsw, s, ca, geom(Vn));
-                }
-            } else if (conv_pf && M == 64 && (ca.kin == 16 || ca.kin == 64)) {
+            if (conv_pf && M == 64 && (ca.kin == 16 || ca.kin == 64)) {
                 if (ca.kin == 64) {
                     if (np == 64) hipLaunchKernelGGL((k_conv_rows_pf<2, 2, 64, EPI>), grd, dim3(256), lds, s, ca, geom(Vn));
                     else hipLaunchKernelGGL((k_conv_rows_pf<2, 1, 64, EPI>), grd, dim3(256), lds, s, ca, geom(Vn));
@@ -320,35 +364,33 @@ struct CNN {
         wa.kin = c.kinp;
         wa.np = c.np;
         wa.kp = c.kpt;
-        int ns = nsplit;
-        bool bias_done = false; // the plane kernel also forms the bias partials
-        if (planes_wgrad && (c.np == 32 || c.np == 64) && (c.kpt == 32 || c.kpt == 64)) {
+        int ns = nsplit, nb = 0; // weight partials, bias partials
+        bool bias_done = false;  // the row kernel also forms the bias partials
+        if (tr_wgrad && (c.np == 32 || c.np == 64) && (c.kpt == 32 || c.kpt == 64)) {
             bias_done = true;
-            WGradPlaneArgs wp;
-            wp.dout = dout;
-            wp.in = wa.in;
-            wp.part = wpart;
-            wp.bpart = bpart;
-            wp.nout = c.nout;
-            wp.ldd = ldd;
-            wp.kin = c.kinp;
-            const long nplanes = (long)B * M;
-            wp.planes_per_block = (int)((nplanes + wgrad_splits - 1) / wgrad_splits);
-            ns = (int)((nplanes + wp.planes_per_block - 1) / wp.planes_per_block);
-            wp.lds_d = wgrad_row_stride(M);
-            wp.lds_i = wgrad_row_stride(M + 16);
-            const int NC = (c.np / 32) * (c.kpt / 32);
-            const size_t stage = sizeof(unsigned short) * ((size_t)c.np * wp.lds_d + (size_t)3 * c.kpt * wp.lds_i);
-            const size_t lds = std::max(stage, NC < 4 ? sizeof(float) * 1024 * 9 * (size_t)NC : (size_t)0);
-            const dim3 grd(ns, 3);
+            WGradTrArgs wt;
+            wt.dout = dout;
+            wt.in = wa.in;
+            wt.part = wpart;
+            wt.bpart = bpart;
+            wt.nout = c.nout;
+            wt.ldd = ldd;
+            wt.kin = c.kinp;
+            const long nrows = (long)B * M * M;
+            wt.rows_per_block = (int)((nrows + wgrad_splits - 1) / wgrad_splits);
+            nb = (int)((nrows + wt.rows_per_block - 1) / wt.rows_per_block);
+            const int wpc = 4 / ((c.np / 32) * (c.kpt / 32));
+            ns = nb * wpc;
+            const size_t lds = std::max<size_t>((size_t)2 * M * 2 * c.np + (size_t)4 * (M + 2) * 2 * c.kpt, 256 * 8 * sizeof(float));
+            const dim3 grd(nb, 3);
             if (c.np == 64 && c.kpt == 64)
-                hipLaunchKernelGGL((k_conv_wgrad_planes<2, 2>), grd, dim3(256), lds, st, wp, geom(V));
+                hipLaunchKernelGGL((k_conv_wgrad_tr<2, 2>), grd, dim3(256), lds, st, wt, geom(V));
             else if (c.np == 64)
-                hipLaunchKernelGGL((k_conv_wgrad_planes<2, 1>), grd, dim3(256), lds, st, wp, geom(V));
+                hipLaunchKernelGGL((k_conv_wgrad_tr<2, 1>), grd, dim3(256), lds, st, wt, geom(V));
             else if (c.kpt == 64)
-                hipLaunchKernelGGL((k_conv_wgrad_planes<1, 2>), grd, dim3(256), lds, st, wp, geom(V));
+                hipLaunchKernelGGL((k_conv_wgrad_tr<1, 2>), grd, dim3(256), lds, st, wt, geom(V));
             else
-                hipLaunchKernelGGL((k_conv_wgrad_planes<1, 1>), grd, dim3(256), lds, st, wp, geom(V));
+                hipLaunchKernelGGL((k_conv_wgrad_tr<1, 1>), grd, dim3(256), lds, st, wt, geom(V));
         } else if (rows_wgrad && (c.np == 32 || c.np == 64) && (c.kpt == 32 || c.kpt == 64)) {
             WGradRowArgs wr;
             wr.dout = dout;
@@ -392,14 +434,14 @@ struct CNN {
             wa.chunk = (wa.chunk + 63) / 64 * 64;
             hipLaunchKernelGGL(k_conv_wgrad, dim3(nsplit, 27), dim3(256), 0, st, wa, geom(V));
         }
-        hipLaunchKernelGGL(k_wgrad_reduce, dim3(256), dim3(256), 0, st, wpart, ns, c.np, c.kpt, c.nout, c.kin,
+        hipLaunchKernelGGL(k_wgrad_reduce, dim3(ceil_div(27L * c.nout * c.kin, 64)), dim3(256), 0, st, wpart, ns, c.np, c.kpt, c.nout, c.kin,
                            g + c.woff);
         if (ldd <= 0 || ldd % 8 != 0 || 2048 % ldd != 0 || c.nout > ldd) {
             set_error("bias gradient: channel stride %d is not a multiple of 8 dividing 2048", ldd);
             return DNS_EINVAL;
         }
         if (bias_done) {
-            hipLaunchKernelGGL(k_bias_reduce, dim3(c.nout), dim3(256), 0, st, bpart, ns, c.nout, g + c.boff);
+            hipLaunchKernelGGL(k_bias_reduce, dim3(c.nout), dim3(256), 0, st, bpart, nb, c.nout, g + c.boff);
         } else {
             hipLaunchKernelGGL(k_bias_grad, dim3(bblocks), dim3(256), 0, st, dout, ldd, c.nout, V, bpart);
             hipLaunchKernelGGL(k_bias_reduce, dim3(c.nout), dim3(256), 0, st, bpart, bblocks, c.nout, g + c.boff);
@@ -527,11 +569,15 @@ struct CNN {
     // stages dataset samples idx[0..nb) into batch slots 0..nb (normalised)
     void stage(const int *idx, int nb)
     {
-        for (int b = 0; b < nb; ++b) {
-            hipLaunchKernelGGL((k_planar_to_bf16<float>), dim3(512), dim3(256), 0, st, ds_u[idx[b]], 3, Vs,
-                               (float)(1.0 / su), x0 + (size_t)b * Vs * 16, 16);
-            hipLaunchKernelGGL(k_planar_to_interleaved, dim3(512), dim3(256), 0, st, ds_t[idx[b]], 6, Vs,
-                               (float)(1.0 / stau), t + (size_t)b * Vs * 6);
+        for (int b0 = 0; b0 < nb; b0 += STAGE_SLOTS) {
+            const int cnt = std::min(STAGE_SLOTS, nb - b0);
+            StagePairs p{};
+            for (int q = 0; q < cnt; ++q) {
+                p.u[q] = ds_u[idx[b0 + q]];
+                p.t[q] = ds_t[idx[b0 + q]];
+            }
+            hipLaunchKernelGGL(k_stage_pairs, dim3(ceil_div(Vs, 256), cnt), dim3(256), 0, st, p, Vs, (float)(1.0 / su),
+                               (float)(1.0 / stau), x0 + (size_t)b0 * Vs * 16, t + (size_t)b0 * Vs * 6);
         }
     }
 
@@ -611,7 +657,7 @@ struct CNN {
         stage(&q, 1);
         DNS_TRY(forward(st, 1));
         float *tmp = reinterpret_cast<float *>(dz[0]); // free between training steps
-        hipLaunchKernelGGL((k_interleaved_to_planar<float>), dim3(512), dim3(256), 0, st, y, 6, Vs, stau, tmp);
+        hipLaunchKernelGGL((k_stress_to_planar<float>), dim3(ceil_div(Vs, 256)), dim3(256), 0, st, y, Vs, stau, tmp);
         DNS_HIP_CHECK(hipMemcpyAsync(tau, tmp, sizeof(float) * 6 * Vs, hipMemcpyDeviceToHost, st));
         DNS_HIP_CHECK(hipStreamSynchronize(st));
         return DNS_OK;
@@ -622,9 +668,9 @@ struct CNN {
     {
         DNS_HIP_CHECK(hipEventRecord(ev_in, st));
         DNS_HIP_CHECK(hipStreamWaitEvent(s, ev_in, 0));
-        hipLaunchKernelGGL((k_planar_to_bf16<T>), dim3(512), dim3(256), 0, s, vel, 3, Vs, (float)(1.0 / su), x0, 16);
+        hipLaunchKernelGGL((k_velocity_to_bf16<T>), dim3(ceil_div(Vs, 256)), dim3(256), 0, s, vel, Vs, (float)(1.0 / su), x0);
         DNS_TRY(forward(s, 1));
-        hipLaunchKernelGGL((k_interleaved_to_planar<T>), dim3(512), dim3(256), 0, s, y, 6, Vs, stau, tau);
+        hipLaunchKernelGGL((k_stress_to_planar<T>), dim3(ceil_div(Vs, 256)), dim3(256), 0, s, y, Vs, stau, tau);
         DNS_HIP_CHECK(hipGetLastError());
         DNS_HIP_CHECK(hipEventRecord(ev_out, s));
         DNS_HIP_CHECK(hipStreamWaitEvent(st, ev_out, 0));
