@@ -126,6 +126,7 @@ template <typename T> struct FVImpl : FVBase {
     size_t ldst = 0;
     int cn_tl = 0, cn_nthr = 256; // x-lines and threads per block of the LDS CN kernel (0: sequential)
     int cn_seg = 0;               // rows per segment of the equal-segment CN kernel (0: not used)
+    int cn_rows = 0;              // rows its segments hold (S·R >= ny)
     int cn_fused = 0;             // the three components in one launch (k_cn_seg3): 1 pressure rows re-read, 2 staged in LDS
     int cn_nl = 1;                // x-lines per thread of the equal-segment CN kernel
     size_t ldscn = 0;
@@ -439,12 +440,16 @@ template <typename T> struct FVImpl : FVBase {
                     thomas_tl = tl;
             }
             if (!thomas_tl) DNS_TRY(dalloc(&Dth, (size_t)g.ldc * ny * nz));
-            // equal segments of R rows (ny = S·R) use k_thomas_seg; DNS_THOMAS=tile keeps k_thomas_tile
+            // segments of R rows, S·R >= ny, use k_thomas_seg; DNS_THOMAS=tile keeps k_thomas_tile
             thomas_seg = 0;
             if (thomas_tl && thomas_nthr == 256 && !(env && !strcmp(env, "tile")) &&
                 (size_t)g.ldc * ny * sizeof(cplx<T>) < ((size_t)1 << 31)) {
-                const int S = thomas_nthr / thomas_tl, R = ny / S;
-                if (ny % S == 0 && (R == 4 || R == 6 || R == 8 || R == 12 || R == 16 || R == 24)) thomas_seg = R;
+                const int S = thomas_nthr / thomas_tl;
+                for (int R : {4, 6, 8, 12, 16, 24})
+                    if (!thomas_seg && S * R >= ny) thomas_seg = R;
+                ldst = (size_t)thomas_nthr * 40 + (size_t)2 * S * thomas_seg * sizeof(double);
+                if (ldst > (size_t)maxlds) thomas_seg = 0;
+                if (!thomas_seg) ldst = (size_t)thomas_nthr * 40 + (size_t)2 * ny * sizeof(double);
             }
             if (imexy && (size_t)6 * ny * sizeof(double) > (size_t)maxlds) {
                 set_error("unsupported grid: implicit y-diffusion coefficients need %zu bytes of LDS",
@@ -470,15 +475,17 @@ template <typename T> struct FVImpl : FVBase {
                     }
                 }
                 if (!cn_tl) DNS_TRY(dalloc(&Dcn, (size_t)N));
-                // equal segments of R rows (ny = S·R) use k_cn_seg; DNS_CN=tile keeps k_cn_tile
+                // segments of R rows, S·R >= ny, use k_cn_seg; DNS_CN=tile keeps k_cn_tile
                 cn_seg = 0;
                 // (its buffer offsets are 32-bit byte offsets within one z plane)
                 if (cn_tl && cn_nthr == 256 && !(envc && !strcmp(envc, "tile")) &&
                     (size_t)nx * ny * sizeof(T) < ((size_t)1 << 31)) {
-                    const int S = cn_nthr / cn_tl, R = ny / S;
-                    if (ny % S == 0 && (R == 8 || R == 16 || R == 24 || R == 32) &&
-                        ldscn + (size_t)ny * sizeof(double) <= (size_t)maxlds)
-                        cn_seg = R;
+                    const int S = cn_nthr / cn_tl;
+                    for (int R : {8, 16, 24, 32})
+                        if (!cn_seg && S * R >= ny &&
+                            (size_t)3 * cn_nthr * sizeof(double) + (size_t)7 * S * R * sizeof(double) <= (size_t)maxlds)
+                            cn_seg = R;
+                    if (cn_seg) cn_rows = S * cn_seg;
                 }
                 // DNS_CN_NL=2: two x-lines per thread (pair accesses, block rows twice
                 // as wide, same segments); one line measured as fast in FP64 and faster
@@ -486,7 +493,7 @@ template <typename T> struct FVImpl : FVBase {
                 cn_nl = 1;
                 if (cn_seg && nx % 2 == 0) {
                     const char *en = getenv("DNS_CN_NL");
-                    const size_t need = (size_t)6 * cn_nthr * sizeof(double) + (size_t)7 * ny * sizeof(double);
+                    const size_t need = (size_t)6 * cn_nthr * sizeof(double) + (size_t)7 * cn_rows * sizeof(double);
                     if (en && atoi(en) == 2 && need <= (size_t)maxlds) {
                         cn_nl = 2;
                         cn_tl *= 2;
@@ -505,7 +512,7 @@ template <typename T> struct FVImpl : FVBase {
                     cn_fused = ef ? atoi(ef) : (sizeof(T) == 8 ? 2 : 0);
                     if (!cn_seg || cn_nl != 1 || cn_fused < 0 || cn_fused > 2) cn_fused = 0;
                     if (cn_fused == 2 &&
-                        (size_t)(3 + cn_seg + 1) * cn_nthr * sizeof(double) + (size_t)7 * ny * sizeof(double) > (size_t)maxlds)
+                        (size_t)(3 + cn_seg + 1) * cn_nthr * sizeof(double) + (size_t)7 * cn_rows * sizeof(double) > (size_t)maxlds)
                         cn_fused = ef ? 1 : 0;
                 }
                 if (cn_tl && !cn_seg && (ny + cn_nthr / cn_tl - 1) / (cn_nthr / cn_tl) > CN_RMAX) {
@@ -930,7 +937,7 @@ template <typename T> struct FVImpl : FVBase {
     // equal-segment CN kernel for component c with R rows per thread
     template <int R, int NL> void cn_seg_launch_nl(int c, dim3 grd, dim3 blk, const CNArgs<T> &a)
     {
-        const size_t lds = (size_t)3 * NL * cn_nthr * sizeof(double) + (size_t)7 * g.ny * sizeof(double);
+        const size_t lds = (size_t)3 * NL * cn_nthr * sizeof(double) + (size_t)7 * cn_rows * sizeof(double);
         if (c == 0) hipLaunchKernelGGL((k_cn_seg<T, 0, R, NL>), grd, blk, lds, st, a, g, cn_tl);
         else if (c == 1) hipLaunchKernelGGL((k_cn_seg<T, 1, R, NL>), grd, blk, lds, st, a, g, cn_tl);
         else hipLaunchKernelGGL((k_cn_seg<T, 2, R, NL>), grd, blk, lds, st, a, g, cn_tl);
@@ -977,7 +984,7 @@ template <typename T> struct FVImpl : FVBase {
             a.rdz = 1.0 / dz;
             const dim3 grd(ceil_div(g.nx, cn_tl), g.nz), blk(cn_nthr);
             const size_t lds = (size_t)(3 + (cn_fused == 2 ? cn_seg + 1 : 0)) * cn_nthr * sizeof(double) +
-                               (size_t)7 * g.ny * sizeof(double);
+                               (size_t)7 * cn_rows * sizeof(double);
             timer.begin(FAM_CN);
             if (cn_fused == 2) {
                 switch (cn_seg) {

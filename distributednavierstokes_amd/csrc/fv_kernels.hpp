@@ -1024,12 +1024,15 @@ __global__ void __launch_bounds__(512) k_thomas_tile(cplx<T> *__restrict__ A, co
     }
 }
 
-// k_thomas_tile for equal segments (ny = S·R): no row needs a bounds test,
-// and the rows of r and of the pivot table are read through buffer
-// resources (one offset register per array for all R rows, a scalar offset
-// per row), all issued before the first use.  Register budget: two blocks
+// k_thomas_tile with segments of exactly R rows (S·R >= ny): no row needs a
+// bounds test, and the rows of r and of the pivot table are read through
+// buffer resources (one offset register per array for all R rows, a scalar
+// offset per row), all issued before the first use.  Rows past the line lie
+// beyond both buffer ranges: they read zero, have zero coefficients, so both
+// recurrences pass them as zeros, and their stores are dropped; the chains
+// walk only the segments that hold rows.  Register budget: two blocks
 // of 256 threads per CU.  Same recurrences, pivots and mean-mode rule.
-// grid (ceil(nxc / TL), nz); LDS 2 ny + 5 blockDim doubles.
+// grid (ceil(nxc / TL), nz); LDS 2 S R + 5 blockDim doubles.
 template <typename T, int R>
 __global__ void __launch_bounds__(256, 2) k_thomas_seg(cplx<T> *__restrict__ A, const double *__restrict__ ip,
                                                        const double *__restrict__ ay, const double *__restrict__ cy,
@@ -1037,11 +1040,11 @@ __global__ void __launch_bounds__(256, 2) k_thomas_seg(cplx<T> *__restrict__ A, 
                                                        double scale, int TL, FVGeom g)
 {
     extern __shared__ unsigned char smem_raw[];
-    const int ny = g.ny, S = blockDim.x / TL;
+    const int ny = g.ny, SR = (int)blockDim.x / TL * R, S = (ny + R - 1) / R; // S: segments with rows
     double2 *Bs = reinterpret_cast<double2 *>(smem_raw); // [S][TL] segment offsets
     double2 *Xin = Bs + blockDim.x;                      // [S][TL] segment inflows
     double *As = reinterpret_cast<double *>(Xin + blockDim.x);
-    double *sa = As + blockDim.x, *sc = sa + ny;
+    double *sa = As + blockDim.x, *sc = sa + SR;
     int bxr, byr;
     xcd_block2(bxr, byr);
     const int kx0 = bxr * TL, kz = byr;
@@ -1067,9 +1070,9 @@ __global__ void __launch_bounds__(256, 2) k_thomas_seg(cplx<T> *__restrict__ A, 
 #pragma unroll
         for (int q = 0; q < R; ++q) x[q] = make_double2((double)ar[q].x * scale, (double)ar[q].y * scale);
     }
-    for (int j = threadIdx.x; j < ny; j += blockDim.x) {
-        sa[j] = ay[j];
-        sc[j] = cy[j];
+    for (int j = threadIdx.x; j < SR; j += blockDim.x) {
+        sa[j] = j < ny ? ay[j] : 0.0;
+        sc[j] = j < ny ? cy[j] : 0.0;
     }
     const bool mean = (lam1[kxl] + lam3[kz]) == 0.0;
     __syncthreads();
@@ -1138,6 +1141,7 @@ __global__ void __launch_bounds__(256, 2) k_thomas_seg(cplx<T> *__restrict__ A, 
     }
     __syncthreads();
     if (!valid) return;
+    if (sg >= S) return; // no rows (nor an inflow)
     const double2 xi = Xin[threadIdx.x];
     double P = 1.0;
 #pragma unroll
@@ -1519,9 +1523,11 @@ __global__ void __launch_bounds__(512) k_cn_tile(CNArgs<T> a, FVGeom g, int TL)
     }
 }
 
-// k_cn_tile for the common case of equal segments: every line's ny rows
-// split into S segments of exactly R rows (ny = S·R), so no row needs a
-// bounds test.  Each thread owns NL neighbouring x-lines (NL = 2: pair
+// k_cn_tile with segments of exactly R rows (S·R >= ny), so no row needs a
+// bounds test: rows past the line lie beyond the plane's buffer range (they
+// read zero, their stores are dropped) and have zero coefficients, so both
+// sweeps pass them as zeros; the chains walk only the segments with rows
+// (384x201x240 FP64, three components: 0.77 ms by k_cn_tile, 0.46 here).  Each thread owns NL neighbouring x-lines (NL = 2: pair
 // accesses of 8 or 16 bytes, a block row of TL lines is TL·sizeof(T) bytes
 // wide) over the R rows of its segment; S = blockDim·NL / TL.  All loads of
 // a chunk of CH rows are issued unconditionally (the row past a line end
@@ -1531,7 +1537,7 @@ __global__ void __launch_bounds__(512) k_cn_tile(CNArgs<T> a, FVGeom g, int TL)
 // k_cn_tile.  Loads go through buffer resources (one offset register per
 // array for all rows) and the register budget is two blocks per CU (three
 // spilled and measured slower).
-// grid (ceil(nx / TL), nz); LDS 7 ny + 3 NL blockDim doubles.
+// grid (ceil(nx / TL), nz); LDS 7 S R + 3 NL blockDim doubles.
 template <typename T, int NL> struct CNVec;
 template <typename T> struct CNVec<T, 1> {
     using type = T;
@@ -1556,18 +1562,20 @@ __global__ void __launch_bounds__(256, 2) k_cn_seg(CNArgs<T> a, FVGeom g, int TL
     using VT = typename CV::type;
     extern __shared__ unsigned char smem_raw[];
     constexpr int CH = R % 8 == 0 ? 8 : R;
-    const int ny = g.ny, TLT = TL / NL, S = blockDim.x / TLT; // threads per block row, segments
+    const int ny = g.ny, TLT = TL / NL;                                  // threads per block row
+    const int SR = (int)blockDim.x / TLT * R, S = (ny + R - 1) / R;      // rows held; segments with rows
     double *As = reinterpret_cast<double *>(smem_raw), *Bs = As + NL * blockDim.x, *Xin = Bs + NL * blockDim.x;
-    double *ca = Xin + NL * blockDim.x, *cb = ca + ny, *cc = cb + ny, *cf = cc + ny, *ci = cf + ny, *cq = ci + ny;
-    double *cr = cq + ny; // 1/Δyu of the normal rows
-    for (int j = threadIdx.x; j < ny; j += blockDim.x) {
-        if (COMP == 1) cr[j] = a.rdyu[j + 1];
-        ca[j] = j == 0 ? 0.0 : a.a[j]; // Dy rows with the couplings past the line ends cut
-        cb[j] = a.b[j];
-        cc[j] = j == ny - 1 ? 0.0 : a.c[j];
-        cf[j] = j == 0 ? 0.0 : a.theta * a.a[j] * a.ip[j];
-        ci[j] = a.ip[j];
-        cq[j] = j == ny - 1 ? 0.0 : -a.cp[j];
+    double *ca = Xin + NL * blockDim.x, *cb = ca + SR, *cc = cb + SR, *cf = cc + SR, *ci = cf + SR, *cq = ci + SR;
+    double *cr = cq + SR; // 1/Δyu of the normal rows
+    for (int j = threadIdx.x; j < SR; j += blockDim.x) {
+        const bool in = j < ny;
+        if (COMP == 1) cr[j] = in ? a.rdyu[j + 1] : 0.0;
+        ca[j] = j == 0 || !in ? 0.0 : a.a[j]; // Dy rows with the couplings past the line ends cut
+        cb[j] = in ? a.b[j] : 0.0;
+        cc[j] = j >= ny - 1 ? 0.0 : a.c[j];
+        cf[j] = j == 0 || !in ? 0.0 : a.theta * a.a[j] * a.ip[j];
+        ci[j] = in ? a.ip[j] : 0.0;
+        cq[j] = j >= ny - 1 ? 0.0 : -a.cp[j];
     }
     const int l = threadIdx.x % TLT, sg = threadIdx.x / TLT;
     int bxr, byr;
@@ -1694,7 +1702,7 @@ __global__ void __launch_bounds__(256, 2) k_cn_seg(CNArgs<T> a, FVGeom g, int TL
         }
     }
     __syncthreads();
-    if (!valid) return;
+    if (!valid || sg >= S) return;
     double xi[NL], P[NL];
 #pragma unroll
     for (int e = 0; e < NL; ++e) {
@@ -1724,7 +1732,7 @@ __global__ void __launch_bounds__(256, 2) k_cn_seg(CNArgs<T> a, FVGeom g, int TL
 // LDS.  The y component uses the normal-row coefficient set, x and z the
 // tangential one: the LDS coefficient rows are restaged between components.
 // Same arithmetic in the same order as k_cn_seg for each component.
-// grid (ceil(nx / TL), nz); LDS 7 ny + (R + 4) blockDim doubles.
+// grid (ceil(nx / TL), nz); LDS 7 S R + (R + 4) blockDim doubles.
 template <typename T> struct CN3Args {
     T *u[3];
     const T *q[3];
@@ -1742,7 +1750,7 @@ __device__ __forceinline__ void cn3_component(const CN3Args<T> &a, const FVGeom 
                                               const double *cr)
 {
     constexpr int CH = R % 8 == 0 ? 8 : R;
-    const int ny = g.ny, S = blockDim.x / TL;
+    const int ny = g.ny, S = (ny + R - 1) / R; // segments with rows
     const int l = threadIdx.x % TL, sg = threadIdx.x / TL;
     int bxr, byr;
     xcd_block2(bxr, byr);
@@ -1859,7 +1867,7 @@ __device__ __forceinline__ void cn3_component(const CN3Args<T> &a, const FVGeom 
         }
     }
     __syncthreads();
-    if (valid) {
+    if (valid && sg < S) {
         const double xi = Xin[threadIdx.x];
         double P = 1.0;
 #pragma unroll
@@ -1874,22 +1882,23 @@ template <typename T, int R, bool PKL>
 __global__ void __launch_bounds__(256, 2) k_cn_seg3(CN3Args<T> a, FVGeom g, int TL)
 {
     extern __shared__ unsigned char smem_raw[];
-    const int ny = g.ny;
+    const int ny = g.ny, SR = (int)blockDim.x / TL * R; // rows held by the block's segments
     double *As = reinterpret_cast<double *>(smem_raw), *Bs = As + blockDim.x, *Xin = Bs + blockDim.x;
-    double *ca = Xin + blockDim.x, *cb = ca + ny, *cc = cb + ny, *cf = cc + ny, *ci = cf + ny, *cq = ci + ny;
-    double *cr = cq + ny;            // 1/Δyu of the normal rows
-    double *pks = cr + ny;           // the threads' pressure rows, R + 1 each
+    double *ca = Xin + blockDim.x, *cb = ca + SR, *cc = cb + SR, *cf = cc + SR, *ci = cf + SR, *cq = ci + SR;
+    double *cr = cq + SR;            // 1/Δyu of the normal rows
+    double *pks = cr + SR;           // the threads' pressure rows, R + 1 each
     auto stage = [&](int set) {
-        for (int j = threadIdx.x; j < ny; j += blockDim.x) {
-            ca[j] = j == 0 ? 0.0 : a.ya[set][j]; // Dy rows with the couplings past the line ends cut
-            cb[j] = a.yb[set][j];
-            cc[j] = j == ny - 1 ? 0.0 : a.yc[set][j];
-            cf[j] = j == 0 ? 0.0 : a.theta * a.ya[set][j] * a.ip[set][j];
-            ci[j] = a.ip[set][j];
-            cq[j] = j == ny - 1 ? 0.0 : -a.cp[set][j];
+        for (int j = threadIdx.x; j < SR; j += blockDim.x) {
+            const bool in = j < ny;
+            ca[j] = j == 0 || !in ? 0.0 : a.ya[set][j]; // Dy rows with the couplings past the line ends cut
+            cb[j] = in ? a.yb[set][j] : 0.0;
+            cc[j] = j >= ny - 1 ? 0.0 : a.yc[set][j];
+            cf[j] = j == 0 || !in ? 0.0 : a.theta * a.ya[set][j] * a.ip[set][j];
+            ci[j] = in ? a.ip[set][j] : 0.0;
+            cq[j] = j >= ny - 1 ? 0.0 : -a.cp[set][j];
         }
     };
-    for (int j = threadIdx.x; j < ny; j += blockDim.x) cr[j] = a.rdyu[j + 1];
+    for (int j = threadIdx.x; j < SR; j += blockDim.x) cr[j] = j < ny ? a.rdyu[j + 1] : 0.0;
     stage(0);
     // this thread's pressure rows j0 .. j0 + R of plane k (past the plane: 0)
     const int l = threadIdx.x % TL, sg = threadIdx.x / TL;
