@@ -1030,7 +1030,8 @@ __global__ void __launch_bounds__(512) k_thomas_tile(cplx<T> *__restrict__ A, co
 // offset per row), all issued before the first use.  Rows past the line lie
 // beyond both buffer ranges: they read zero, have zero coefficients, so both
 // recurrences pass them as zeros, and their stores are dropped; the chains
-// walk only the segments that hold rows.  Register budget: two blocks
+// walk only the segments that hold rows (the others get no inflow; whatever
+// they compute is dropped).  Register budget: two blocks
 // of 256 threads per CU.  Same recurrences, pivots and mean-mode rule.
 // grid (ceil(nxc / TL), nz); LDS 2 S R + 5 blockDim doubles.
 template <typename T, int R>
@@ -1070,10 +1071,11 @@ __global__ void __launch_bounds__(256, 2) k_thomas_seg(cplx<T> *__restrict__ A, 
 #pragma unroll
         for (int q = 0; q < R; ++q) x[q] = make_double2((double)ar[q].x * scale, (double)ar[q].y * scale);
     }
-    for (int j = threadIdx.x; j < SR; j += blockDim.x) {
-        sa[j] = j < ny ? ay[j] : 0.0;
-        sc[j] = j < ny ? cy[j] : 0.0;
+    for (int j = threadIdx.x; j < ny; j += blockDim.x) {
+        sa[j] = ay[j];
+        sc[j] = cy[j];
     }
+    for (int j = ny + threadIdx.x; j < SR; j += blockDim.x) sa[j] = sc[j] = 0.0;
     const bool mean = (lam1[kxl] + lam3[kz]) == 0.0;
     __syncthreads();
     // forward sweep d'_j = −a_j ip_j d'_{j−1} + ip_j r_j (row 0: no coupling; 0 for the mean mode)
@@ -1141,7 +1143,6 @@ __global__ void __launch_bounds__(256, 2) k_thomas_seg(cplx<T> *__restrict__ A, 
     }
     __syncthreads();
     if (!valid) return;
-    if (sg >= S) return; // no rows (nor an inflow)
     const double2 xi = Xin[threadIdx.x];
     double P = 1.0;
 #pragma unroll
@@ -1567,16 +1568,16 @@ __global__ void __launch_bounds__(256, 2) k_cn_seg(CNArgs<T> a, FVGeom g, int TL
     double *As = reinterpret_cast<double *>(smem_raw), *Bs = As + NL * blockDim.x, *Xin = Bs + NL * blockDim.x;
     double *ca = Xin + NL * blockDim.x, *cb = ca + SR, *cc = cb + SR, *cf = cc + SR, *ci = cf + SR, *cq = ci + SR;
     double *cr = cq + SR; // 1/Δyu of the normal rows
-    for (int j = threadIdx.x; j < SR; j += blockDim.x) {
-        const bool in = j < ny;
-        if (COMP == 1) cr[j] = in ? a.rdyu[j + 1] : 0.0;
-        ca[j] = j == 0 || !in ? 0.0 : a.a[j]; // Dy rows with the couplings past the line ends cut
-        cb[j] = in ? a.b[j] : 0.0;
-        cc[j] = j >= ny - 1 ? 0.0 : a.c[j];
-        cf[j] = j == 0 || !in ? 0.0 : a.theta * a.a[j] * a.ip[j];
-        ci[j] = in ? a.ip[j] : 0.0;
-        cq[j] = j >= ny - 1 ? 0.0 : -a.cp[j];
+    for (int j = threadIdx.x; j < ny; j += blockDim.x) {
+        if (COMP == 1) cr[j] = a.rdyu[j + 1];
+        ca[j] = j == 0 ? 0.0 : a.a[j]; // Dy rows with the couplings past the line ends cut
+        cb[j] = a.b[j];
+        cc[j] = j == ny - 1 ? 0.0 : a.c[j];
+        cf[j] = j == 0 ? 0.0 : a.theta * a.a[j] * a.ip[j];
+        ci[j] = a.ip[j];
+        cq[j] = j == ny - 1 ? 0.0 : -a.cp[j];
     }
+    for (int j = ny + threadIdx.x; j < SR; j += blockDim.x) ca[j] = cb[j] = cc[j] = cf[j] = ci[j] = cq[j] = cr[j] = 0.0;
     const int l = threadIdx.x % TLT, sg = threadIdx.x / TLT;
     int bxr, byr;
     xcd_block2(bxr, byr);
@@ -1702,7 +1703,7 @@ __global__ void __launch_bounds__(256, 2) k_cn_seg(CNArgs<T> a, FVGeom g, int TL
         }
     }
     __syncthreads();
-    if (!valid || sg >= S) return;
+    if (!valid) return;
     double xi[NL], P[NL];
 #pragma unroll
     for (int e = 0; e < NL; ++e) {
@@ -1867,7 +1868,7 @@ __device__ __forceinline__ void cn3_component(const CN3Args<T> &a, const FVGeom 
         }
     }
     __syncthreads();
-    if (valid && sg < S) {
+    if (valid) {
         const double xi = Xin[threadIdx.x];
         double P = 1.0;
 #pragma unroll
@@ -1888,17 +1889,17 @@ __global__ void __launch_bounds__(256, 2) k_cn_seg3(CN3Args<T> a, FVGeom g, int 
     double *cr = cq + SR;            // 1/Δyu of the normal rows
     double *pks = cr + SR;           // the threads' pressure rows, R + 1 each
     auto stage = [&](int set) {
-        for (int j = threadIdx.x; j < SR; j += blockDim.x) {
-            const bool in = j < ny;
-            ca[j] = j == 0 || !in ? 0.0 : a.ya[set][j]; // Dy rows with the couplings past the line ends cut
-            cb[j] = in ? a.yb[set][j] : 0.0;
-            cc[j] = j >= ny - 1 ? 0.0 : a.yc[set][j];
-            cf[j] = j == 0 || !in ? 0.0 : a.theta * a.ya[set][j] * a.ip[set][j];
-            ci[j] = in ? a.ip[set][j] : 0.0;
-            cq[j] = j >= ny - 1 ? 0.0 : -a.cp[set][j];
+        for (int j = threadIdx.x; j < ny; j += blockDim.x) {
+            ca[j] = j == 0 ? 0.0 : a.ya[set][j]; // Dy rows with the couplings past the line ends cut
+            cb[j] = a.yb[set][j];
+            cc[j] = j == ny - 1 ? 0.0 : a.yc[set][j];
+            cf[j] = j == 0 ? 0.0 : a.theta * a.ya[set][j] * a.ip[set][j];
+            ci[j] = a.ip[set][j];
+            cq[j] = j == ny - 1 ? 0.0 : -a.cp[set][j];
         }
     };
-    for (int j = threadIdx.x; j < SR; j += blockDim.x) cr[j] = j < ny ? a.rdyu[j + 1] : 0.0;
+    for (int j = threadIdx.x; j < ny; j += blockDim.x) cr[j] = a.rdyu[j + 1];
+    for (int j = ny + threadIdx.x; j < SR; j += blockDim.x) ca[j] = cb[j] = cc[j] = cf[j] = ci[j] = cq[j] = cr[j] = 0.0;
     stage(0);
     // this thread's pressure rows j0 .. j0 + R of plane k (past the plane: 0)
     const int l = threadIdx.x % TL, sg = threadIdx.x / TL;

@@ -19,6 +19,7 @@ template <typename T> struct X2Args {
     double *vpart;   // one partial of max Σ_c |v_c| per block, or null
     const cplx<T> *tw, *twx; // exp(-2πi t/N), t < N; exp(-2πi t/n), t <= N
     int n, K, mode;
+    int nlines;      // lines of P (n² of phys and tau, which only whole grids pass)
 };
 
 }  // namespace dns

@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(256, 2) k_sp_x2(X2Args<T> a)
     for (int e = threadIdx.x; e < N; e += blockDim.x) twx[e] = a.twx[e];
     __syncthreads();
 
-    const int n = a.n, K = a.K, nlines = n * n, sz = (int)sizeof(cplx<T>);
+    const int n = a.n, K = a.K, nlines = a.nlines, sz = (int)sizeof(cplx<T>);
     const int L0 = __builtin_amdgcn_readfirstlane((xcd_block(blockIdx.x, gridDim.x) * nwv + wv) * LPW);
     const int nl = __builtin_amdgcn_readfirstlane(max(0, min(LPW, nlines - L0))); // lines of this wavefront
     const bool mine = lg < nl;

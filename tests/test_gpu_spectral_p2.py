@@ -47,3 +47,18 @@ def test_p2_transforms_rhs_step_products(n, kcut, T):
         check(lib().dns_spec_products(s.handle))
         check(lib().dns_spec_get_products(s.handle, dptr(sg)))
         assert np.abs(sg - sig).max() <= tol * np.abs(sig).max()
+
+
+def test_slab_step_216():
+    """A grid whose product pencils exceed the memory-side cache takes the z
+    and x passes in 64-row slabs (here 64, 64, 64 and 24): step and max Σ|v|
+    against the oracle."""
+    n = 216
+    s = dns.spectral_setup(n=n, visc=5e-3)
+    o = OracleSpectral(SpectralProblem(n=n, visc=5e-3))
+    ref = o.randomfield(totalenergy=0.5, kpeak=4, seed=1)
+    got = ref.copy(order="F")
+    vr = o.step(ref, 2e-3)
+    vm = dns.spectral_step_(got, s, 2e-3)
+    assert abs(vm - vr) <= 1e-12 * vr
+    assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()
