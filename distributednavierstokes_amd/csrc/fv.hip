@@ -72,12 +72,11 @@ constexpr int RED_BLOCKS = 1024;
 // Scratch of the allocation-free CFL loop (dns_fv_advance_cfl_noalloc), one
 // file-scope array per GPU (160 KiB, held until the process ends).  Layout in
 // doubles: [0] Δt, [1] t, [2] step counter (an int in its first 4 bytes),
-// [NOALLOC_PART, +3·512) per-block maxima of the CFL reduction,
-// [NOALLOC_RED, +3) reduced maxima, [NOALLOC_LOG, +NOALLOC_MAX_STEPS) the
+// [NOALLOC_PART, +3·512) per-block maxima of the CFL reduction, [NOALLOC_LOG, +NOALLOC_MAX_STEPS) the
 // Δt log.  Host code never names the array in a launch or copy: it uses the
 // address hipGetSymbolAddress gave for the current device (noalloc_scratch).
 constexpr int NOALLOC_MAX_STEPS = 16384;
-constexpr size_t NOALLOC_PART = 256, NOALLOC_RED = 2048, NOALLOC_LOG = 4096;
+constexpr size_t NOALLOC_PART = 256, NOALLOC_LOG = 4096;
 constexpr size_t NOALLOC_DOUBLES = NOALLOC_LOG + NOALLOC_MAX_STEPS;
 static __device__ __align__(256) double scratch[NOALLOC_DOUBLES];
 
@@ -1350,6 +1349,22 @@ template <typename T> struct FVImpl : FVBase {
         return DNS_OK;
     }
 
+    // Δt on the device from the pressure-gradient partials: one launch up to
+    // 8192 of them, else a first level of up to 512 blocks into mid
+    void launch_cfl_dt(double *mid, double diff, double cflv, double tend, double *t, double *dt, double *log, int *step)
+    {
+        const double *part = upart;
+        int n = nb_pgrad;
+        if (n > 8192) {
+            const int G = std::min(512, n / 1024);
+            hipLaunchKernelGGL(k_max_mid, dim3(G), dim3(NTHR), 0, st, upart, n, 3, mid);
+            part = mid;
+            n = G;
+        }
+        hipLaunchKernelGGL(k_cfl_dt, dim3(1), dim3(n > 256 ? 1024 : 256), 0, st, part, n, dx, dymin, dz, diff, cflv, tend, t,
+                           dt, log, step);
+    }
+
     int read_back(size_t count)
     {
         DNS_HIP_CHECK(hipMemcpyAsync(pinned, redout, sizeof(double) * count, hipMemcpyDeviceToHost, st));
@@ -1417,7 +1432,6 @@ template <typename T> struct FVImpl : FVBase {
         const double eps = 2.220446049250313e-16;
         const double invdy2 = 1 / (dymin * dymin);
         const double diff = 1 / (2 * visc * (1 / (dx * dx) + invdy2 + 1 / (dz * dz)) + eps);
-        const int G = std::min(512, std::max(1, nb_pgrad / 1024));
         for (; done < nsteps; ++done) {
             const int key = u[0] == ubuf0 ? 0 : 1;
             if (!gcfl[key] || gcfl_key[key][0] != cflv || gcfl_key[key][1] != tend) {
@@ -1427,10 +1441,7 @@ template <typename T> struct FVImpl : FVBase {
                 }
                 hipGraph_t graph = nullptr;
                 DNS_HIP_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-                hipLaunchKernelGGL(k_max_mid, dim3(G), dim3(NTHR), 0, st, upart, nb_pgrad, 3, red);
-                hipLaunchKernelGGL(k_max_final, dim3(1), dim3(NTHR), 0, st, red, G, 3, redout);
-                hipLaunchKernelGGL(k_cfl_dt, dim3(1), dim3(1), 0, st, redout, dx, dymin, dz, diff, cflv, tend, dtime,
-                                   ddt, dlog, dstep);
+                launch_cfl_dt(red, diff, cflv, tend, dtime, ddt, dlog, dstep);
                 mom_dtp = ddt;
                 const int rc = step_launch(0.0);
                 mom_dtp = nullptr;
@@ -1521,18 +1532,14 @@ template <typename T> struct FVImpl : FVBase {
             return DNS_OK;
         }
         double *sdt = noalloc_s, *stime = noalloc_s + 1, *spart = noalloc_s + NOALLOC_PART,
-               *sred = noalloc_s + NOALLOC_RED, *slog = noalloc_s + NOALLOC_LOG;
+               *slog = noalloc_s + NOALLOC_LOG;
         int *sstep = reinterpret_cast<int *>(noalloc_s + 2);
         const int step0 = done;
         hipLaunchKernelGGL(k_noalloc_start, dim3(1), dim3(1), 0, st, noalloc_s, t);
         const double eps = 2.220446049250313e-16;
         const double diff = 1 / (2 * visc * (1 / (dx * dx) + 1 / (dymin * dymin) + 1 / (dz * dz)) + eps);
-        const int G = std::min(512, std::max(1, nb_pgrad / 1024));
         for (; done < nsteps; ++done) {
-            hipLaunchKernelGGL(k_max_mid, dim3(G), dim3(NTHR), 0, st, upart, nb_pgrad, 3, spart);
-            hipLaunchKernelGGL(k_max_final, dim3(1), dim3(NTHR), 0, st, spart, G, 3, sred);
-            hipLaunchKernelGGL(k_cfl_dt, dim3(1), dim3(1), 0, st, sred, dx, dymin, dz, diff, cflv, tend, stime, sdt,
-                               slog, sstep);
+            launch_cfl_dt(spart, diff, cflv, tend, stime, sdt, slog, sstep);
             mom_dtp = sdt;
             const int rc = step_launch(0.0);
             mom_dtp = nullptr;
@@ -1558,10 +1565,14 @@ template <typename T> struct FVImpl : FVBase {
     {
         if (umax_valid) {
             // partial maxima left by the pressure-gradient pass that produced u,
-            // reduced in two levels (up to 512 blocks, then one)
-            const int G = std::min(512, std::max(1, nb_pgrad / 1024));
-            hipLaunchKernelGGL(k_max_mid, dim3(G), dim3(NTHR), 0, st, upart, nb_pgrad, 3, red);
-            hipLaunchKernelGGL(k_max_final, dim3(1), dim3(NTHR), 0, st, red, G, 3, redout);
+            // reduced in two levels (up to 512 blocks, then one), few of them in one
+            if (nb_pgrad > 2048) {
+                const int G = std::min(512, std::max(1, nb_pgrad / 1024));
+                hipLaunchKernelGGL(k_max_mid, dim3(G), dim3(NTHR), 0, st, upart, nb_pgrad, 3, red);
+                hipLaunchKernelGGL(k_max_final, dim3(1), dim3(NTHR), 0, st, red, G, 3, redout);
+            } else {
+                hipLaunchKernelGGL(k_max_final, dim3(1), dim3(NTHR), 0, st, upart, nb_pgrad, 3, redout);
+            }
         } else {
             const int nb = std::min(RED_BLOCKS, ceil_div(N, NTHR));
             hipLaunchKernelGGL((k_maxabs3<T>), dim3(nb), dim3(NTHR), 0, st, u[0], u[1], u[2], N, red);
