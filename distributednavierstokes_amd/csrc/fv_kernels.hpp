@@ -292,7 +292,8 @@ __global__ void __launch_bounds__(256) k_momentum_slab(MomentumArgs<T> a, FVGeom
 // are fixed for the whole march, so a plane costs a few adds per load.  The
 // loads of plane k+3 are issued before plane k is computed, and plane k+2
 // (issued one plane earlier) lands in LDS after it: two planes in flight per
-// thread.  The old q values are read before the plane loads.  Rows outside the wall follow the ldc/ldf ghost rules.
+// thread.  The old q values are read before the plane loads, with QA one plane
+// earlier.  Rows outside the wall follow the ldc/ldf ghost rules.
 // Grid (ceil(nx/64), ceil(ny/8), ceil(nz/zc)) of 256 threads, XCD-ordered;
 // LDS 3 planes × 3 components × 10 rows × (64 + 2V) + metric rows.
 template <typename T> struct LZ {
@@ -306,7 +307,7 @@ template <typename T> struct LZ {
     static constexpr int PL = NROW * P;               // one plane slot
 };
 
-template <typename T, bool READ_Q, bool WRITE_V>
+template <typename T, bool READ_Q, bool WRITE_V, bool QA = false>
 __global__ void __launch_bounds__(256) k_momentum_lz(MomentumArgs<T> a, FVGeom g, int zc)
 {
     resolve_dt(a);
@@ -420,6 +421,22 @@ __global__ void __launch_bounds__(256) k_momentum_lz(MomentumArgs<T> a, FVGeom g
         if (hlane) dst[hdst] = hsgn == T(0) ? T(0) : hsgn * hr;
     };
 
+    // old q of the plane being updated; QA: loaded one plane ahead
+    const int tx = tid & 63, ty = __builtin_amdgcn_readfirstlane(tid >> 6);
+    T qn[2][3];
+    auto load_q = [&](int k, T (&qd)[2][3]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int j = y0 + ty + 4 * h;
+            const size_t c = (size_t)(x0 + tx) + (size_t)g.nx * j + plane * k;
+            qd[h][0] = qd[h][1] = qd[h][2] = T(0);
+            if (READ_Q && tx < w && j < g.ny) {
+                qd[h][0] = ld_stream(a.qx + c, true);
+                if (!(g.wall && j == g.ny - 1)) qd[h][1] = ld_stream(a.qy + c, true);
+                qd[h][2] = ld_stream(a.qz + c, true);
+            }
+        }
+    };
     {
         // the first planes in flight together (issued and landed one by one,
         // three load latencies stood before every march: eight steps of
@@ -429,30 +446,25 @@ __global__ void __launch_bounds__(256) k_momentum_lz(MomentumArgs<T> a, FVGeom g
         issue(k0 - 1, vB, hB);
         issue(k0, vC, hC);
         issue(k0 + 1, vD, hD);
+        if (QA) load_q(k0, qn);
         if (k0 + 1 < kend) issue(k0 + 2, vA, hA);
         land(0, vB, hB);
         land(1, vC, hC);
         land(2, vD, hD);
     }
     __syncthreads();
-    const int tx = tid & 63, ty = __builtin_amdgcn_readfirstlane(tid >> 6);
     int sM = 0, s0 = 1, sP = 2;
     // one plane: old q values, the loads of plane k+3, the update of plane k,
     // then plane k+2 (in cur) lands in the slot plane k−1 leaves
     auto plane_step = [&](int k, VT (&cur)[L::NI], T &curh, VT (&nxt)[L::NI], T &nxth) {
         const int i = x0 + tx;
         T qo[2][3];
+        if (!QA) load_q(k, qn);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int j = y0 + ty + 4 * h;
-            const size_t c = (size_t)i + (size_t)g.nx * j + plane * k;
-            qo[h][0] = qo[h][1] = qo[h][2] = T(0);
-            if (READ_Q && tx < w && j < g.ny) {
-                qo[h][0] = ld_stream(a.qx + c, true);
-                if (!(g.wall && j == g.ny - 1)) qo[h][1] = ld_stream(a.qy + c, true);
-                qo[h][2] = ld_stream(a.qz + c, true);
-            }
-        }
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) qo[h][c] = qn[h][c];
+        if (QA && k + 1 < kend) load_q(k + 1, qn);
         if (k + 2 < kend) issue(k + 3, nxt, nxth);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
