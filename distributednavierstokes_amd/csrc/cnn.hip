@@ -1,7 +1,7 @@
 // Host side of the sub-filter-stress CNN: a 4-layer 3×3×3 periodic CNN
 // (3 → 64 → 64 → 64 → 6 channels, erf-GELU) on M³ LES grids, trained with
 // Adam on filtered-DNS pairs held on the GPU; BF16 weights and activations
-// with FP32 accumulation (v_mfma_f32_32x32x8_bf16).  C ABI: dns_cnn_*.
+// with FP32 accumulation (v_mfma_f32_32x32x16_bf16).  C ABI: dns_cnn_*.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -218,13 +218,13 @@ struct CNN {
         DNS_TRY(dalloc(&y, (size_t)V * 6));
         DNS_TRY(dalloc(&t, (size_t)V * 6));
         nsplit = (int)std::max<long>(1, std::min<long>(64, V / 4096));
-        // the row-staged weight-gradient kernel splits the B·M² x-rows over at most 256 blocks
+        // the row-staged weight-gradient kernels split the B·M² x-rows over at most 256 blocks
         row_wgrad = !mfma_k8 && M % 16 == 0 && M <= 256;
         const char *envw = getenv("DNS_CNN_WGRAD");
         rows_wgrad = row_wgrad && M <= 64 && envw && !strcmp(envw, "rows");
-        tr_wgrad = row_wgrad && M <= 64 && !(envw && (!strcmp(envw, "rows") || !strcmp(envw, "row16")));
+        tr_wgrad = !mfma_k8 && M <= 64 && !(envw && (!strcmp(envw, "rows") || !strcmp(envw, "row16")));
         if (const char *es = getenv("DNS_CNN_WSPLIT")) wgrad_splits = std::max(1, std::min(256, atoi(es)));
-        const int nsplit16 = row_wgrad ? (int)std::min<long>(256, (long)B * M * M) : 0;
+        const int nsplit16 = row_wgrad || tr_wgrad ? (int)std::min<long>(256, (long)B * M * M) : 0;
         DNS_TRY(dalloc(&wpart, (size_t)std::max(nsplit, nsplit16) * 27 * 64 * 64));
         DNS_TRY(dalloc(&bpart, (size_t)64 * bblocks));
         DNS_TRY(dalloc(&lpart, kLossBlocks));
@@ -251,7 +251,7 @@ struct CNN {
     bool mfma_k8 = false;
     bool row_wgrad = false; // k_conv_wgrad16 (M % 16 == 0) instead of k_conv_wgrad
     bool rows_wgrad = false;   // k_conv_wgrad_rows (M % 16 == 0, M <= 64); DNS_CNN_WGRAD=rows
-    bool tr_wgrad = false;     // k_conv_wgrad_tr (M % 16 == 0, M <= 64), the default
+    bool tr_wgrad = false;     // k_conv_wgrad_tr (M <= 64), the default
     // row splits of k_conv_wgrad_tr: × 3 dz, the blocks of one round at two per
     // CU (DNS_CNN_WSPLIT, sweep)
     int wgrad_splits = 170;
@@ -283,10 +283,12 @@ struct CNN {
             }
             return;
         }
-        // The plane kernel wherever its rows fit the LDS (M up to 176 or so);
-        // measured against k_conv_rows (M = 32) and k_conv16 (other M), ms per
-        // training step: see conv_plane in the table of DNS_CNN_CONV below.
-        if (conv_pf && conv_wlds && (ca.kin == 16 || ca.kin == 64) && (np == 32 || np == 64) &&
+        // The plane kernel wherever its rows fit the LDS (M up to 176 or so)
+        // and the batch the grid's z extent; against k_conv_rows (M = 32, 64)
+        // and k_conv16 (other M), ms per two training steps: 16 × 64³
+        // 16.7 / 32.0, 4 × 48³ 2.45 / 6.30, 4 × 32³ 1.00 / 1.69; five LES
+        // steps of 36³ 2.40 / 5.86, 80³ 10.3 / 23.7.
+        if (conv_pf && conv_wlds && Vn / Vs <= 65535 && (ca.kin == 16 || ca.kin == 64) && (np == 32 || np == 64) &&
             conv_plane_lds(M, np, ca.kin) <= max_lds) {
             if (M == 64) conv_plane<64, EPI>(ca, np, Vn, s);
             else if (M == 32) conv_plane<32, EPI>(ca, np, Vn, s);
@@ -381,7 +383,8 @@ struct CNN {
             nb = (int)((nrows + wt.rows_per_block - 1) / wt.rows_per_block);
             const int wpc = 4 / ((c.np / 32) * (c.kpt / 32));
             ns = nb * wpc;
-            const size_t lds = std::max<size_t>((size_t)2 * M * 2 * c.np + (size_t)4 * (M + 2) * 2 * c.kpt, 256 * 8 * sizeof(float));
+            const int MP = (M + 15) & ~15;
+            const size_t lds = std::max<size_t>((size_t)2 * MP * 2 * c.np + (size_t)4 * (MP + 2) * 2 * c.kpt, 256 * 8 * sizeof(float));
             const dim3 grd(nb, 3);
             if (c.np == 64 && c.kpt == 64)
                 hipLaunchKernelGGL((k_conv_wgrad_tr<2, 2>), grd, dim3(256), lds, st, wt, geom(V));

@@ -576,8 +576,9 @@ __device__ __forceinline__ void conv_epilogue_lds(const f32x16 (&acc)[MB][NB], c
 // Weights: at KIN = 64 each offset's block is loaded an offset ahead into a
 // double-buffered LDS copy (one barrier per offset); at KIN = 16 the blocks of
 // all 27 offsets (27 NP 32 bytes) are staged once and no barrier separates
-// the offsets (with four MFMAs per offset and barrier the 3 → 64 and 6 → 64
-// layers ran at 17 % MFMA busy, 0.60 ms for 16 × 64³).  Both operands are kept
+// the offsets.  Writing the results as whole lines through LDS
+// (conv_epilogue_lds) took the 3 → 64 and 6 → 64 layers of 16 × 64³ from 0.58
+// to 0.45 ms, 64 → 64 forward from 0.99 to 0.91.  Both operands are kept
 // so that the lanes of a fragment read spread over the banks: rows of
 // KIN + 8 halves at KIN = 64, two planes of 8 channels at KIN = 16.
 // Products are accumulated in the order dz, dy, dx, k for every voxel.
@@ -1111,14 +1112,19 @@ __global__ void __launch_bounds__(256) k_conv_wgrad_rows(WGradRowArgs a, ConvGeo
 // one is read) and a ring of four input rows y−1 … y+2 (row y' in slot
 // (y' + 1) mod 4) with one halo voxel on each side, so a row costs one
 // barrier; its global loads are in flight during the MFMAs of the two rows
-// before (one row ahead left the kernel waiting on them: 1.30 ms).  64-channel rows (128 bytes) swap their 64-byte halves on every
+// before (one row ahead left the kernel waiting on them: 1.30 ms per 64 → 64
+// layer, two 0.97–1.02; 3 → 64 0.61 and 64 → 6 0.51, from 1.66 and 1.33).
+// 64-channel rows (128 bytes) swap their 64-byte halves on every
 // second pair of voxels: the 4 voxels × 64 bytes that 32 lanes read then
 // cover all banks once.
 //
 // Wave w takes the (n-tile, k-tile) pair w mod NT·KT and the 16-voxel slices
 // s ≡ w / (NT·KT) (mod 4 / (NT·KT)); waves sharing a pair write partials of
 // their own: part[blockIdx.x · WPC + w / (NT·KT)][o][n][k].
-// Needs M % 16 == 0, M <= 64, NT = np/32 and KT = kp/32 in {1, 2}, ldd and
+// Rows of M % 16 != 0 voxels are filled up to MP with zeros; two training
+// steps against the voxel-tile kernel (k_conv_wgrad): 16 × 8³ 0.66 / 5.9 ms,
+// 4 × 24³ 0.87 / 6.7, 12 × 40³ 4.1 / 34.7.
+// Needs M <= 64 (two 16-byte pieces of a row per thread), NT = np/32 and KT = kp/32 in {1, 2}, ldd and
 // kin multiples of 8.
 struct WGradTrArgs {
     const unsigned short *dout; // [V][ldd]
@@ -1149,10 +1155,10 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeo
     constexpr int NP = 32 * NT, KP = 32 * KT, NC = NT * KT, WPC = 4 / NC;
     constexpr int RD = 2 * NP, RI = 2 * KP; // bytes per voxel of the two row kinds
     constexpr int PMAX = 2;                 // 16-byte pieces of a row per thread (M <= 64)
-    const int M = g.M, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    unsigned char *sd = smem_raw;                // [2][M][NP]
-    unsigned char *si = smem_raw + 2 * M * RD;   // [4][M + 2][KP], voxel x at x + 1
-    const int SLOT = (M + 2) * RI;
+    const int M = g.M, MP = (M + 15) & ~15, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    unsigned char *sd = smem_raw;                // [2][MP][NP]
+    unsigned char *si = smem_raw + 2 * MP * RD;  // [4][MP + 2][KP], voxel x at x + 1
+    const int SLOT = (MP + 2) * RI;
     const int dzi = blockIdx.y;
     const int combo = wave % NC, sg = wave / NC, nt = combo % NT, kt = combo / NT;
     const int nrows = g.B * M * M;
@@ -1186,7 +1192,7 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeo
             const int e = tid + 256 * q;
             if (e >= nd) continue;
             const int v = e / pcd, c = e - v * pcd;
-            *reinterpret_cast<u32x4 *>(sd + buf * M * RD + at(v, 16 * c, RD)) = pd[q];
+            *reinterpret_cast<u32x4 *>(sd + buf * MP * RD + at(v, 16 * c, RD)) = pd[q];
             if (dobias) {
 #pragma unroll
                 for (int w = 0; w < 4; ++w) {
@@ -1219,9 +1225,9 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeo
         }
     };
 
-    // channels past ldd and kin stay zero
-    if (a.ldd < NP || a.kin < KP)
-        for (int e = tid; e < (2 * M * RD + 4 * SLOT) / 16; e += 256)
+    // channels past ldd and kin and voxels past M stay zero
+    if (a.ldd < NP || a.kin < KP || MP != M)
+        for (int e = tid; e < (2 * MP * RD + 4 * SLOT) / 16; e += 256)
             reinterpret_cast<u32x4 *>(smem_raw)[e] = u32x4{0u, 0u, 0u, 0u};
 
     f32x16 acc[9];
@@ -1238,8 +1244,8 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeo
         const int yn = min(y + 2, y1 - 1); // rows past the range: loaded, not stored
         load_d(qd, p * M + yn);
         load_i(qi, p, yn + 1);
-        const unsigned char *da = sd + cur * M * RD + offa;
-        for (int s = sg; s < M / 16; s += WPC) {
+        const unsigned char *da = sd + cur * MP * RD + offa;
+        for (int s = sg; s < MP / 16; s += WPC) {
             const bf16x8 av = lds_read_tr(da + 16 * s * RD, 4 * RD);
 #pragma unroll
             for (int dyi = 0; dyi < 3; ++dyi) {
