@@ -367,7 +367,7 @@ struct CNN {
         wa.np = c.np;
         wa.kp = c.kpt;
         int ns = nsplit, nb = 0; // weight partials, bias partials
-        bool bias_done = false;  // the row kernel also forms the bias partials
+        bool bias_done = false;  // the weight kernel also forms the bias partials
         if (tr_wgrad && (c.np == 32 || c.np == 64) && (c.kpt == 32 || c.kpt == 64)) {
             bias_done = true;
             WGradTrArgs wt;
@@ -437,18 +437,16 @@ struct CNN {
             wa.chunk = (wa.chunk + 63) / 64 * 64;
             hipLaunchKernelGGL(k_conv_wgrad, dim3(nsplit, 27), dim3(256), 0, st, wa, geom(V));
         }
-        hipLaunchKernelGGL(k_wgrad_reduce, dim3(ceil_div(27L * c.nout * c.kin, 64)), dim3(256), 0, st, wpart, ns, c.np, c.kpt, c.nout, c.kin,
-                           g + c.woff);
         if (ldd <= 0 || ldd % 8 != 0 || 2048 % ldd != 0 || c.nout > ldd) {
             set_error("bias gradient: channel stride %d is not a multiple of 8 dividing 2048", ldd);
             return DNS_EINVAL;
         }
-        if (bias_done) {
-            hipLaunchKernelGGL(k_bias_reduce, dim3(c.nout), dim3(256), 0, st, bpart, nb, c.nout, g + c.boff);
-        } else {
-            hipLaunchKernelGGL(k_bias_grad, dim3(bblocks), dim3(256), 0, st, dout, ldd, c.nout, V, bpart);
-            hipLaunchKernelGGL(k_bias_reduce, dim3(c.nout), dim3(256), 0, st, bpart, bblocks, c.nout, g + c.boff);
+        if (!bias_done) {
+            nb = bblocks;
+            hipLaunchKernelGGL(k_bias_grad, dim3(nb), dim3(256), 0, st, dout, ldd, c.nout, V, bpart);
         }
+        hipLaunchKernelGGL(k_wgrad_reduce, dim3(ceil_div(27L * c.nout * c.kin, 64) + c.nout), dim3(256), 0, st, wpart,
+                           ns, c.np, c.kpt, c.nout, c.kin, g + c.woff, bpart, nb, g + c.boff);
         DNS_HIP_CHECK(hipGetLastError());
         return DNS_OK;
     }
@@ -509,16 +507,19 @@ struct CNN {
         aa.m = m;
         aa.v = v;
         aa.g = g;
-        aa.count = (long)nparam;
+        aa.count = (int)nparam;
         aa.lr = lr;
         aa.b1 = b1;
         aa.b2 = b2;
         aa.eps = eps;
         aa.c1 = (float)(1.0 / (1.0 - std::pow((double)b1, adam_t)));
         aa.c2 = (float)(1.0 / (1.0 - std::pow((double)b2, adam_t)));
+        for (int l = 0; l < 4; ++l) {
+            const CNNLayer &c = L[l];
+            aa.layer[l] = {(int)c.woff, 27 * c.nout * c.kin, c.nout, c.kin, c.np, c.kinp, c.kpt, c.noutp, c.W, c.WT};
+        }
         timer.begin(2);
-        hipLaunchKernelGGL(k_adam, dim3(256), dim3(256), 0, st, aa);
-        DNS_TRY(pack());
+        hipLaunchKernelGGL(k_adam, dim3(ceil_div((long)nparam, 256)), dim3(256), 0, st, aa);
         timer.end(2);
         DNS_HIP_CHECK(hipGetLastError());
         return DNS_OK;

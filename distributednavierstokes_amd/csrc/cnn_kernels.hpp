@@ -1315,10 +1315,28 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeo
 // order, eight loads in flight each, and the four sums are added pairwise
 // (fixed order).  One thread per element with four loads in flight left the
 // reads latency-bound: 29-43 µs per layer for 170 splits, 75 MB.
+// The nout blocks past those sum the bias partials bpart[c][x], x < nb, one
+// channel each: strided FP64 partial sums, then a tree in LDS (a launch of its
+// own took 4.8 µs per layer).
 __global__ void __launch_bounds__(256) k_wgrad_reduce(const float *part, int nsplit, int np, int kp, int nout, int kin,
-                                                      float *grad)
+                                                      float *grad, const float *bpart, int nb, float *bgrad)
 {
     __shared__ double s[4][64];
+    const int wblocks = (27 * nout * kin + 63) / 64;
+    if ((int)blockIdx.x >= wblocks) {
+        const int c = blockIdx.x - wblocks;
+        double *sb = s[0];
+        double acc = 0;
+        for (int q = threadIdx.x; q < nb; q += blockDim.x) acc += bpart[(size_t)c * nb + q];
+        sb[threadIdx.x] = acc;
+        __syncthreads();
+        for (int w = 128; w > 0; w >>= 1) {
+            if (threadIdx.x < w) sb[threadIdx.x] += sb[threadIdx.x + w];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) bgrad[c] = (float)sb[0];
+        return;
+    }
     const int total = 27 * nout * kin, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t = blockIdx.x * 64 + lane, tc = min(t, total - 1);
     const int k = tc % kin, n = (tc / kin) % nout, o = tc / (kin * nout);
@@ -1375,23 +1393,6 @@ __global__ void __launch_bounds__(256) k_bias_grad(const unsigned short *dout, i
     }
 }
 
-// One block of 256 threads per channel (grid nout): strided FP64 partial
-// sums, then a tree in LDS (fixed order).
-__global__ void __launch_bounds__(256) k_bias_reduce(const float *part, int nblocks, int nout, float *grad)
-{
-    __shared__ double s[256];
-    const int c = blockIdx.x;
-    double acc = 0;
-    for (int q = threadIdx.x; q < nblocks; q += blockDim.x) acc += part[(size_t)c * nblocks + q];
-    s[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && c < nout) grad[c] = (float)s[0];
-}
-
 // MSE loss over `nout` channels: dy = 2(y − t)/(V nout) (BF16, padded to
 // ldd channels with zeros), per-block partial sums of (y − t)².
 __global__ void __launch_bounds__(256) k_mse(const float *y, const float *t, int nout, long V, unsigned short *dy,
@@ -1434,25 +1435,44 @@ __global__ void __launch_bounds__(256) k_mse(const float *y, const float *t, int
 }
 
 // Adam on FP32 masters; refreshes the BF16 forward (W[o][n][k], n padded to
-// np) and transposed (WT[o][k][n], k padded to kpt) copies.  bias tail of
-// each layer is stored after its weights in the flat parameter vector.
+// np) and transposed (WT[o][k][n], k padded to kpt) copies in the same pass
+// (their padding stays as k_pack_weights wrote it; a pack launch per layer
+// took 27 µs of a 475 µs step of 4 × 32³).  The bias tail of each layer is
+// stored after its weights in the flat parameter vector.
+struct AdamLayer {
+    int woff, nw; // weights of the layer in the flat vector: [woff, woff + nw), order [o][n][k]
+    int nout, kin, np, kinp, kpt, noutp;
+    unsigned short *W, *WT;
+};
 struct AdamArgs {
     float *w, *m, *v;
     const float *g;
-    long count;
+    int count;
     float lr, b1, b2, eps, c1, c2; // c1 = 1/(1−b1^t), c2 = 1/(1−b2^t)
+    AdamLayer layer[4];
 };
 
 __global__ void __launch_bounds__(256) k_adam(AdamArgs a)
 {
-    for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < a.count; t += (long)gridDim.x * blockDim.x) {
-        const float g = a.g[t];
-        const float m = a.b1 * a.m[t] + (1.f - a.b1) * g;
-        const float v = a.b2 * a.v[t] + (1.f - a.b2) * g * g;
-        a.m[t] = m;
-        a.v[t] = v;
-        const float mh = m * a.c1, vh = v * a.c2;
-        a.w[t] -= a.lr * mh / (sqrtf(vh) + a.eps);
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= a.count) return;
+    const float g = a.g[t];
+    const float m = a.b1 * a.m[t] + (1.f - a.b1) * g;
+    const float v = a.b2 * a.v[t] + (1.f - a.b2) * g * g;
+    a.m[t] = m;
+    a.v[t] = v;
+    const float mh = m * a.c1, vh = v * a.c2;
+    const float w = a.w[t] - a.lr * mh / (sqrtf(vh) + a.eps);
+    a.w[t] = w;
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+        const AdamLayer &c = a.layer[l];
+        const int e = t - c.woff;
+        if (e < 0 || e >= c.nw) continue;
+        const int k = e % c.kin, n = (e / c.kin) % c.nout, o = e / (c.kin * c.nout);
+        const unsigned short h = f2bf(w);
+        c.W[(o * c.np + n) * c.kinp + k] = h;
+        c.WT[(o * c.kpt + k) * c.noutp + n] = h;
     }
 }
 
