@@ -263,13 +263,23 @@ struct CNN {
     {
         const dim3 grd((unsigned)ceil_div((long)M * M, 256), (unsigned)M, (unsigned)(Vn / Vs)), blk(256);
         const size_t lds = conv_plane_lds(M, np, ca.kin);
-        if (ca.kin == 64) {
-            if (np == 64) hipLaunchKernelGGL((k_conv_plane<MC, 2, 64, EPI>), grd, blk, lds, s, ca, geom(Vn));
-            else hipLaunchKernelGGL((k_conv_plane<MC, 1, 64, EPI>), grd, blk, lds, s, ca, geom(Vn));
-        } else {
-            if (np == 64) hipLaunchKernelGGL((k_conv_plane<MC, 2, 16, EPI>), grd, blk, lds, s, ca, geom(Vn));
-            else hipLaunchKernelGGL((k_conv_plane<MC, 1, 16, EPI>), grd, blk, lds, s, ca, geom(Vn));
-        }
+        constexpr int NB = EPI == 1 ? 1 : 2; // 6 outputs, else 64
+        if (ca.kin == 64) hipLaunchKernelGGL((k_conv_plane<MC, NB, 64, EPI>), grd, blk, lds, s, ca, geom(Vn));
+        else hipLaunchKernelGGL((k_conv_plane<MC, NB, 16, EPI>), grd, blk, lds, s, ca, geom(Vn));
+    }
+    // The output convolution where no backward pass follows: k_conv_out sums
+    // dx last, so its results differ from k_conv_plane's in the last FP32 bits,
+    // and a gradient would see them where a BF16 dy rounds the other way.
+    bool conv_out(const ConvArgs &ca, long Vn, hipStream_t s)
+    {
+        const size_t lds = M <= 256 ? conv_out_lds(M, ca.nout) : 0;
+        if (!conv_pf || mfma_k8 || ca.kin != 64 || ca.nout > CO_NMAX || M > 256 || Vn / Vs > 65535 || lds > max_lds) return false;
+        const dim3 grd((unsigned)ceil_div(M, conv_out_rows(M)), (unsigned)M, (unsigned)(Vn / Vs));
+        if (M == 64) hipLaunchKernelGGL((k_conv_out<64>), grd, dim3(256), lds, s, ca, geom(Vn));
+        else if (M == 32) hipLaunchKernelGGL((k_conv_out<32>), grd, dim3(256), lds, s, ca, geom(Vn));
+        else if (M == 16) hipLaunchKernelGGL((k_conv_out<16>), grd, dim3(256), lds, s, ca, geom(Vn));
+        else hipLaunchKernelGGL((k_conv_out<0>), grd, dim3(256), lds, s, ca, geom(Vn));
+        return true;
     }
     template <int EPI> void conv(const ConvArgs &ca, int np, long Vn, hipStream_t s)
     {
@@ -288,7 +298,7 @@ struct CNN {
         // and k_conv16 (other M), ms per two training steps: 16 × 64³
         // 16.7 / 32.0, 4 × 48³ 2.45 / 6.30, 4 × 32³ 1.00 / 1.69; five LES
         // steps of 36³ 2.40 / 5.86, 80³ 10.3 / 23.7.
-        if (conv_pf && conv_wlds && Vn / Vs <= 65535 && (ca.kin == 16 || ca.kin == 64) && (np == 32 || np == 64) &&
+        if (conv_pf && conv_wlds && Vn / Vs <= 65535 && (ca.kin == 16 || ca.kin == 64) && np == (EPI == 1 ? 32 : 64) &&
             conv_plane_lds(M, np, ca.kin) <= max_lds) {
             if (M == 64) conv_plane<64, EPI>(ca, np, Vn, s);
             else if (M == 32) conv_plane<32, EPI>(ca, np, Vn, s);
@@ -325,8 +335,10 @@ struct CNN {
         }
     }
 
-    // forward of the first nb batch slots of x0; the FP32 output lands in y (nb M³ × 6)
-    int forward(hipStream_t s, int nb)
+    // forward of the first nb batch slots of x0; the FP32 output lands in y
+    // (nb M³ × 6); the layers' z (half of the bytes a hidden layer writes)
+    // only where a backward pass follows (keep_z)
+    int forward(hipStream_t s, int nb, bool keep_z = false)
     {
         const long Vn = (long)nb * Vs;
         for (int l = 0; l < 4; ++l) {
@@ -341,13 +353,13 @@ struct CNN {
             ca.sign = 1;
             if (l < 3) {
                 ca.out = a[l];
-                ca.zbuf = z[l];
+                ca.zbuf = keep_z ? z[l] : nullptr;
                 ca.ldo = 64;
                 conv<0>(ca, c.np, Vn, s);
             } else {
                 ca.yout = y;
                 ca.ldo = 6;
-                conv<1>(ca, c.np, Vn, s);
+                if (keep_z || !conv_out(ca, Vn, s)) conv<1>(ca, c.np, Vn, s);
             }
         }
         DNS_HIP_CHECK(hipGetLastError());
@@ -614,7 +626,7 @@ struct CNN {
             }
             stage(idx.data(), B);
             timer.begin(0);
-            DNS_TRY(forward(st, B));
+            DNS_TRY(forward(st, B, true));
             timer.end(0);
             DNS_TRY(backward(dl + it));
             DNS_TRY(adam(lr, b1, b2, eps));
@@ -817,7 +829,7 @@ int dns_cnn_loss_grad(dns_cnn *h, const float *x, const float *tgt, double *loss
     DNS_HIP_CHECK(hipMemcpyAsync(tmp, x, sizeof(float) * c.V * 3, hipMemcpyHostToDevice, c.st));
     DNS_HIP_CHECK(hipMemcpyAsync(c.t, tgt, sizeof(float) * c.V * 6, hipMemcpyHostToDevice, c.st));
     hipLaunchKernelGGL(k_to_bf16, dim3(1024), dim3(256), 0, c.st, tmp, 3, 1.0f, c.V, c.x0, 16);
-    DNS_TRY(c.forward(c.st, c.B));
+    DNS_TRY(c.forward(c.st, c.B, true));
     DNS_TRY(c.backward(c.lval));
     double l = 0;
     DNS_TRY(c.read_scalar(c.lval, &l));
