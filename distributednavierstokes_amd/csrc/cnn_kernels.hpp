@@ -588,7 +588,9 @@ inline size_t conv_plane_rows(int M) { return M % 256 == 0 || 256 % M == 0 ? std
 inline size_t conv_plane_lds(int M, int np, int kin)
 {
     const size_t vox = std::min(conv_plane_rows(M), (size_t)M + 2) * M;
-    const size_t work = kin == 16 ? 32 * vox + (size_t)27 * np * 32 : (vox + 2 * np) * 2 * (kin + 8);
+    const bool pipe = M == 16 || M == 32 || M == 64;
+    const size_t work = kin == 16 ? 32 * vox + (size_t)27 * np * 32
+                                  : vox * 2 * (kin + 8) + (pipe ? (size_t)3 * np * 2 * kin : (size_t)2 * np * 2 * (kin + 8));
     return std::max(work, (size_t)4 * 32 * (np + 8) * sizeof(float)); // the epilogue's four areas
 }
 
@@ -597,7 +599,8 @@ __global__ void __launch_bounds__(256) k_conv_plane(ConvArgs a, ConvGeom g)
 {
     extern __shared__ unsigned char smem_raw[];
     unsigned short *sa = reinterpret_cast<unsigned short *>(smem_raw);
-    constexpr bool WALL = KIN == 16; // all weights staged once
+    constexpr bool WALL = KIN == 16;         // all weights staged once
+    constexpr bool PIPE = !WALL && MC != 0;  // fragments one k step ahead, three weight buffers
     constexpr int MB = 2, KST = KIN / 16, KC8 = KIN / 8, NP = 32 * NB, KS = KIN + 8;
     const int M = MC ? MC : g.M, MM = M * M;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -670,7 +673,10 @@ __global__ void __launch_bounds__(256) k_conv_plane(ConvArgs a, ConvGeom g)
 #pragma unroll
         for (int i = 0; i < WPI; ++i) {
             const int e = tid + 256 * i;
-            if (NPW % 256 == 0 || e < NPW) *reinterpret_cast<u32x4 *>(sw + (buf * NP + e / KC8) * KS + 8 * (e % KC8)) = wr[i];
+            const int n = e / KC8, c8 = e % KC8;
+            if (NPW % 256 == 0 || e < NPW)
+                *reinterpret_cast<u32x4 *>(PIPE ? sw + (buf * NP + n) * KIN + 8 * (c8 ^ ((n >> 1) & 7))
+                                                : sw + (buf * NP + n) * KS + 8 * c8) = wr[i];
         }
     };
     bf16x8 zp[MB][2 * NB]; // in flight during the last dz plane
@@ -687,7 +693,24 @@ __global__ void __launch_bounds__(256) k_conv_plane(ConvArgs a, ConvGeom g)
         loadw(0);
         storew(0);
         loadw(1);
+        if (PIPE) {
+            storew(1);
+            loadw(2);
+        }
     }
+    // PIPE: fragments of k step t = 4 o + ks; (32 nb + row) rows of 8 pieces,
+    // piece 2 ks + h of row n at position (2 ks + h) ^ (n / 2 mod 8)
+    bf16x8 fa[2][MB], fw[2][NB];
+    const int wsw = KIN * row + 8 * (h ^ ((row >> 1) & 7));
+    auto frags = [&](int t) __attribute__((always_inline)) {
+        const int o = t / KST, ks = t % KST, q = o % 9;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+            fw[t & 1][nb] = *reinterpret_cast<const bf16x8 *>(sw + ((o % 3) * NP + 32 * nb) * KIN + (wsw ^ (16 * ks)));
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+            fa[t & 1][mb] = *reinterpret_cast<const bf16x8 *>(sa + base[mb][q % 3] + sign * (q / 3 - 1) * vstep + 16 * ks);
+    };
 #pragma unroll
     for (int dzi = 0; dzi < 3; ++dzi) {
         if (WALL && dzi > 0) __syncthreads(); // (else the last offset's barrier)
@@ -704,6 +727,30 @@ __global__ void __launch_bounds__(256) k_conv_plane(ConvArgs a, ConvGeom g)
         if constexpr (MC != 0)
             if (dzi < 2) fetch_rows(dzi + 1);
         if (EPI == 2 && dzi == 2) conv_load_z<MB, NB>(zp, vox, a, lane);
+        if constexpr (PIPE) {
+            frags(9 * KST * dzi);
+#pragma unroll
+            for (int q = 0; q < 9; ++q) {
+                const int o = q + 9 * dzi;
+                // (this buffer was last read in offset o − 1)
+                if (o + 2 < 27) storew((o + 2) % 3);
+                if (o + 3 < 27) loadw(o + 3);
+#pragma unroll
+                for (int ks = 0; ks < KST; ++ks) {
+                    const int t = KST * o + ks;
+                    if (q < 8 || ks + 1 < KST) frags(t + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb)
+                            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[t & 1][nb], fa[t & 1][mb], acc[mb][nb], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                __syncthreads();
+            }
+            continue;
+        }
 #pragma unroll
         for (int q = 0; q < 9; ++q) {
             const int o = q + 9 * dzi, cur = o & 1;
