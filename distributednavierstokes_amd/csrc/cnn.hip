@@ -223,7 +223,7 @@ struct CNN {
         const char *envw = getenv("DNS_CNN_WGRAD");
         rows_wgrad = row_wgrad && M <= 64 && envw && !strcmp(envw, "rows");
         tr_wgrad = !mfma_k8 && M <= 64 && !(envw && (!strcmp(envw, "rows") || !strcmp(envw, "row16")));
-        if (const char *es = getenv("DNS_CNN_WSPLIT")) wgrad_splits = std::max(1, std::min(256, atoi(es)));
+        if (const char *es = getenv("DNS_CNN_WSPLIT")) wgrad_splits = fold_splits = std::max(1, std::min(256, atoi(es)));
         const int nsplit16 = row_wgrad || tr_wgrad ? (int)std::min<long>(256, (long)B * M * M) : 0;
         DNS_TRY(dalloc(&wpart, (size_t)std::max(nsplit, nsplit16) * 27 * 64 * 64));
         DNS_TRY(dalloc(&bpart, (size_t)64 * bblocks));
@@ -253,8 +253,11 @@ struct CNN {
     bool rows_wgrad = false;   // k_conv_wgrad_rows (M % 16 == 0, M <= 64); DNS_CNN_WGRAD=rows
     bool tr_wgrad = false;     // k_conv_wgrad_tr (M <= 64), the default
     // row splits of k_conv_wgrad_tr: × 3 dz, the blocks of one round at two per
-    // CU (DNS_CNN_WSPLIT, sweep)
-    int wgrad_splits = 170;
+    // CU (64 → 64) or three (folded dx: two training steps of 16 × 64³
+    // 15.95 ms with 170, 15.70 with 256); at least 16 / 32 rows per block, so
+    // that a small batch does not spend its time on the partial sums (8 × 16³
+    // 0.60 -> 0.57 ms).  DNS_CNN_WSPLIT: both limits, for sweeps
+    int wgrad_splits = 170, fold_splits = 256;
     bool row_conv = false;  // k_conv_rows (M = 32 or 64) instead of k_conv16; DNS_CNN_CONV=direct disables
     bool conv_pf = false;   // k_conv_plane (k_conv_rows_pf with DNS_CNN_WLDS=0); DNS_CNN_CONV=rows selects k_conv_rows
     bool conv_wlds = true;  // weights shared through LDS; DNS_CNN_WLDS=0 streams them per wavefront (M = 64)
@@ -380,7 +383,7 @@ struct CNN {
         wa.kp = c.kpt;
         int ns = nsplit, nb = 0; // weight partials, bias partials
         bool bias_done = false;  // the weight kernel also forms the bias partials
-        if (tr_wgrad && (c.np == 32 || c.np == 64) && (c.kpt == 32 || c.kpt == 64)) {
+        if (tr_wgrad && (c.np == 64 || (c.np == 32 && c.nout <= 8)) && (c.kpt == 64 || (c.kpt == 32 && c.kin <= 8)) && c.np + c.kpt > 64) {
             bias_done = true;
             WGradTrArgs wt;
             wt.dout = dout;
@@ -391,21 +394,22 @@ struct CNN {
             wt.ldd = ldd;
             wt.kin = c.kinp;
             const long nrows = (long)B * M * M;
-            wt.rows_per_block = (int)((nrows + wgrad_splits - 1) / wgrad_splits);
+            const bool fold = c.np != 64 || c.kpt != 64;
+            const long splits = std::max(1L, std::min<long>(fold ? fold_splits : wgrad_splits, nrows / (fold ? 32 : 16)));
+            wt.rows_per_block = (int)((nrows + splits - 1) / splits);
             nb = (int)((nrows + wt.rows_per_block - 1) / wt.rows_per_block);
             const int wpc = 4 / ((c.np / 32) * (c.kpt / 32));
             ns = nb * wpc;
             const int MP = (M + 15) & ~15;
             const size_t lds = std::max<size_t>((size_t)2 * MP * 2 * c.np + (size_t)4 * (MP + 2) * 2 * c.kpt, 256 * 8 * sizeof(float));
             const dim3 grd(nb, 3);
+            // (64 → 64, 64 → 6, 3 → 64)
             if (c.np == 64 && c.kpt == 64)
-                hipLaunchKernelGGL((k_conv_wgrad_tr<2, 2>), grd, dim3(256), lds, st, wt, geom(V));
-            else if (c.np == 64)
-                hipLaunchKernelGGL((k_conv_wgrad_tr<2, 1>), grd, dim3(256), lds, st, wt, geom(V));
+                hipLaunchKernelGGL((k_conv_wgrad_tr<2, 2, 0>), grd, dim3(256), lds, st, wt, geom(V));
             else if (c.kpt == 64)
-                hipLaunchKernelGGL((k_conv_wgrad_tr<1, 2>), grd, dim3(256), lds, st, wt, geom(V));
+                hipLaunchKernelGGL((k_conv_wgrad_tr<1, 2, 1>), grd, dim3(256), lds, st, wt, geom(V));
             else
-                hipLaunchKernelGGL((k_conv_wgrad_tr<1, 1>), grd, dim3(256), lds, st, wt, geom(V));
+                hipLaunchKernelGGL((k_conv_wgrad_tr<2, 1, 2>), grd, dim3(256), lds, st, wt, geom(V));
         } else if (rows_wgrad && (c.np == 32 || c.np == 64) && (c.kpt == 32 || c.kpt == 64)) {
             WGradRowArgs wr;
             wr.dout = dout;

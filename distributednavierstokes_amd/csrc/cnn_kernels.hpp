@@ -1286,6 +1286,14 @@ __global__ void __launch_bounds__(256) k_conv_wgrad_rows(WGradRowArgs a, ConvGeo
 // Rows of M % 16 != 0 voxels are filled up to MP with zeros; two training
 // steps against the voxel-tile kernel (k_conv_wgrad): 16 × 8³ 0.66 / 5.9 ms,
 // 4 × 24³ 0.87 / 6.7, 12 × 40³ 4.1 / 34.7.
+//
+// FOLD: the narrow operand of the first and last layers (3 input or 6 output
+// channels, at most 8) is staged three times, shifted by dx, as 24 of 32
+// channels, so one MFMA covers the three dx (FOLD = 1: output gradient,
+// E[x][8 d + n] = dout[x − (d − 1)][n]; FOLD = 2: input, E[x][8 d + c] =
+// in[x + d − 1][c]) and the nine accumulators become three (16 × 64³: 64 → 6
+// 579 -> 396 µs, 3 → 64 492 -> 278; barriers and load latency per row are what
+// is left).
 // Needs M <= 64 (two 16-byte pieces of a row per thread), NT = np/32 and KT = kp/32 in {1, 2}, ldd and
 // kin multiples of 8.
 struct WGradTrArgs {
@@ -1310,13 +1318,15 @@ __device__ __forceinline__ bf16x8 lds_read_tr(const unsigned char *p, int second
     return __builtin_bit_cast(bf16x8, v);
 }
 
-template <int NT, int KT>
-__global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeom g)
+template <int NT, int KT, int FOLD>
+__global__ void __launch_bounds__(256, FOLD ? 3 : 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeom g)
 {
     extern __shared__ unsigned char smem_raw[];
     constexpr int NP = 32 * NT, KP = 32 * KT, NC = NT * KT, WPC = 4 / NC;
     constexpr int RD = 2 * NP, RI = 2 * KP; // bytes per voxel of the two row kinds
     constexpr int PMAX = 2;                 // 16-byte pieces of a row per thread (M <= 64)
+    constexpr int PD = FOLD == 1 ? 1 : PMAX, PI = FOLD == 2 ? 1 : PMAX, NA = FOLD ? 3 : 9;
+    static_assert(FOLD == 0 || (FOLD == 1 ? NT == 1 : KT == 1), "the folded operand has one tile");
     const int M = g.M, MP = (M + 15) & ~15, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     unsigned char *sd = smem_raw;                // [2][MP][NP]
     unsigned char *si = smem_raw + 2 * MP * RD;  // [4][MP + 2][KP], voxel x at x + 1
@@ -1338,23 +1348,35 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeo
     for (int d = 0; d < 3; ++d) offb[d] = at(vx + d, 2 * (32 * kt + ch), RI);
 
     // row pieces: piece e is 8 channels (16 bytes) of voxel e / (channels / 8)
-    const int pcd = a.ldd / 8, pci = a.kin / 8, nd = M * pcd, ni = M * pci;
+    // (of a folded operand only the first 8 channels)
+    const int pcd = FOLD == 1 ? 1 : a.ldd / 8, pci = FOLD == 2 ? 1 : a.kin / 8, nd = M * pcd, ni = M * pci;
+    const int stepd = FOLD == 1 ? a.ldd : 8, stepi = FOLD == 2 ? a.kin : 8; // halves between pieces
+    // the three places of a folded voxel's channels
+    auto store3 = [&](unsigned char *p, int v, int dir, const u32x4 &w) __attribute__((always_inline)) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            int x = v + dir * (d - 1);
+            x = x < 0 ? M - 1 : x >= M ? 0 : x;
+            *reinterpret_cast<u32x4 *>(p + 64 * x + 16 * d) = w;
+        }
+    };
     float bsum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     const bool dobias = dzi == 1;
     // (pieces past the row read its last one again: no branch around the
     // loads, so the waits for one row's pieces leave the next row's in flight)
-    auto load_d = [&](u32x4 (&pd)[PMAX], int r) __attribute__((always_inline)) {
+    auto load_d = [&](u32x4 (&pd)[PD], int r) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < PMAX; ++q)
-            pd[q] = *reinterpret_cast<const u32x4 *>(a.dout + ((size_t)r * nd + min(tid + 256 * q, nd - 1)) * 8);
+        for (int q = 0; q < PD; ++q)
+            pd[q] = *reinterpret_cast<const u32x4 *>(a.dout + ((size_t)r * nd + min(tid + 256 * q, nd - 1)) * stepd);
     };
-    auto store_d = [&](const u32x4 (&pd)[PMAX], int buf) __attribute__((always_inline)) {
+    auto store_d = [&](const u32x4 (&pd)[PD], int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < PMAX; ++q) {
+        for (int q = 0; q < PD; ++q) {
             const int e = tid + 256 * q;
             if (e >= nd) continue;
             const int v = e / pcd, c = e - v * pcd;
-            *reinterpret_cast<u32x4 *>(sd + buf * MP * RD + at(v, 16 * c, RD)) = pd[q];
+            if constexpr (FOLD == 1) store3(sd + buf * MP * RD, v, 1, pd[q]);
+            else *reinterpret_cast<u32x4 *>(sd + buf * MP * RD + at(v, 16 * c, RD)) = pd[q];
             if (dobias) {
 #pragma unroll
                 for (int w = 0; w < 4; ++w) {
@@ -1365,21 +1387,25 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeo
         }
     };
     // input row yin (−1 … M) of plane z + dz of the sample of plane p
-    auto load_i = [&](u32x4 (&pi)[PMAX], int p, int yin) __attribute__((always_inline)) {
+    auto load_i = [&](u32x4 (&pi)[PI], int p, int yin) __attribute__((always_inline)) {
         const int z = p % M, zs = z + dzi - 1, zw = zs < 0 ? zs + M : zs >= M ? zs - M : zs;
         const int yw = yin < 0 ? yin + M : yin >= M ? yin - M : yin;
         const size_t row = (size_t)(p - z + zw) * M + yw;
 #pragma unroll
-        for (int q = 0; q < PMAX; ++q)
-            pi[q] = *reinterpret_cast<const u32x4 *>(a.in + (row * ni + min(tid + 256 * q, ni - 1)) * 8);
+        for (int q = 0; q < PI; ++q)
+            pi[q] = *reinterpret_cast<const u32x4 *>(a.in + (row * ni + min(tid + 256 * q, ni - 1)) * stepi);
     };
-    auto store_i = [&](const u32x4 (&pi)[PMAX], int yin) __attribute__((always_inline)) {
+    auto store_i = [&](const u32x4 (&pi)[PI], int yin) __attribute__((always_inline)) {
         unsigned char *slot = si + ((yin + 1) & 3) * SLOT;
 #pragma unroll
-        for (int q = 0; q < PMAX; ++q) {
+        for (int q = 0; q < PI; ++q) {
             const int e = tid + 256 * q;
             if (e >= ni) continue;
             const int v = e / pci, c = e - v * pci;
+            if constexpr (FOLD == 2) {
+                store3(slot + RI, v, -1, pi[q]);
+                continue;
+            }
             *reinterpret_cast<u32x4 *>(slot + at(v + 1, 16 * c, RI)) = pi[q];
             // the periodic halo: voxel 0 again behind the row, voxel M−1 before it
             if (v == 0) *reinterpret_cast<u32x4 *>(slot + at(M + 1, 16 * c, RI)) = pi[q];
@@ -1392,16 +1418,16 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeo
         for (int e = tid; e < (2 * MP * RD + 4 * SLOT) / 16; e += 256)
             reinterpret_cast<u32x4 *>(smem_raw)[e] = u32x4{0u, 0u, 0u, 0u};
 
-    f32x16 acc[9];
+    f32x16 acc[NA];
 #pragma unroll
-    for (int t = 0; t < 9; ++t)
+    for (int t = 0; t < NA; ++t)
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[t][q] = 0.0f;
 
     // one row: LDS holds its output gradient and input rows y−1 … y+1, (pd, pi)
     // the next output-gradient row and input row y+2 (in flight since the
     // row before), (qd, qi) receive those of the row after
-    auto row_step = [&](u32x4 (&pd)[PMAX], u32x4 (&pi)[PMAX], u32x4 (&qd)[PMAX], u32x4 (&qi)[PMAX], int p, int y, int y1,
+    auto row_step = [&](u32x4 (&pd)[PD], u32x4 (&pi)[PI], u32x4 (&qd)[PD], u32x4 (&qi)[PI], int p, int y, int y1,
                         int cur) __attribute__((always_inline)) {
         const int yn = min(y + 2, y1 - 1); // rows past the range: loaded, not stored
         load_d(qd, p * M + yn);
@@ -1412,6 +1438,10 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeo
 #pragma unroll
             for (int dyi = 0; dyi < 3; ++dyi) {
                 const unsigned char *bi = si + ((y + dyi) & 3) * SLOT + 16 * s * RI; // row y + dyi − 1
+                if constexpr (FOLD != 0) {
+                    acc[dyi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, lds_read_tr(bi + offb[1], 4 * RI), acc[dyi], 0, 0, 0);
+                    continue;
+                }
                 bf16x8 bv[3];
 #pragma unroll
                 for (int d = 0; d < 3; ++d) bv[d] = lds_read_tr(bi + offb[d], 4 * RI);
@@ -1429,16 +1459,16 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeo
     for (int r = r0; r < r1;) {
         // the rows of one plane
         const int p = r / M, y0 = r - p * M, y1 = min(M, y0 + r1 - r);
-        u32x4 pd[PMAX], pi[PMAX], qd[PMAX], qi[PMAX];
+        u32x4 pd[PD], pi[PI], qd[PD], qi[PI], ri[PI];
         __syncthreads();
         load_d(pd, r);
         load_i(pi, p, y0 - 1);
         load_i(qi, p, y0);
-        load_i(qd, p, y0 + 1);
+        load_i(ri, p, y0 + 1);
         store_d(pd, 0);
         store_i(pi, y0 - 1);
         store_i(qi, y0);
-        store_i(qd, y0 + 1);
+        store_i(ri, y0 + 1);
         load_d(pd, p * M + min(y0 + 1, y1 - 1));
         load_i(pi, p, min(y0 + 2, M));
         __syncthreads();
@@ -1463,11 +1493,17 @@ __global__ void __launch_bounds__(256, 2) k_conv_wgrad_tr(WGradTrArgs a, ConvGeo
     const size_t pbase = ((size_t)blockIdx.x * WPC + sg) * 27 + 9 * dzi;
     const int row = lane & 31, h = lane >> 5;
 #pragma unroll
-    for (int t = 0; t < 9; ++t)
+    for (int t = 0; t < NA; ++t)
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
             const int i = 8 * (q >> 2) + 4 * h + (q & 3);
-            a.part[((pbase + t) * NP + 32 * nt + i) * KP + 32 * kt + row] = acc[t][q];
+            if constexpr (FOLD == 0) {
+                a.part[((pbase + t) * NP + 32 * nt + i) * KP + 32 * kt + row] = acc[t][q];
+            } else if constexpr (FOLD == 1) { // row i = 8 dx + n
+                if (q < 12) a.part[((pbase + 3 * t + (q >> 2)) * NP + (i & 7)) * KP + 32 * kt + row] = acc[t][q];
+            } else { // column 8 dx + c
+                if (row < 24) a.part[((pbase + 3 * t + (row >> 3)) * NP + 32 * nt + i) * KP + (row & 7)] = acc[t][q];
+            }
         }
 }
 
