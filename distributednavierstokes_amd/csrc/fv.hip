@@ -652,9 +652,11 @@ template <typename T> struct FVImpl : FVBase {
     }
 
     // ---------------------------------------------------------- kernels
-    int launch_momentum(T **uu, T **vv, double Ac, double dt, double B, bool write_v)
+    // psi: uu is not yet corrected by −∇psi (fused stages, stage_fused())
+    int launch_momentum(T **uu, T **vv, double Ac, double dt, double B, bool write_v, const T *psi = nullptr)
     {
         MomentumArgs<T> a;
+        a.psi = psi;
         a.ux = uu[0];
         a.uy = uu[1];
         a.uz = uu[2];
@@ -683,13 +685,15 @@ template <typename T> struct FVImpl : FVBase {
         timer.begin(FAM_MOM);
         const bool rq = Ac != 0.0;
         if (momentum_kind == 5) {
-            // z chunks: the longest power-of-two march up to 32 planes that still
-            // gives one full round of resident blocks (3 per CU in FP64, 6 in FP32)
-            // over 256 CUs (measured: longer marches win until the grid stops
-            // filling the chip; a partial last round costs a whole round)
             const int nbx = ceil_div(g.nx, 64), nby = ceil_div(g.ny, 8);
-            const int zc = momentum_zc();
+            const int zc = momentum_zc(psi != nullptr);
             dim3 grd(nbx, nby, ceil_div(g.nz, zc));
+            if (psi) {
+                hipLaunchKernelGGL((k_momentum_lz<T, true, true, sizeof(T) == 4, true>), grd, dim3(256), 0, st, a, g, zc);
+                timer.end(FAM_MOM);
+                DNS_HIP_CHECK(hipGetLastError());
+                return DNS_OK;
+            }
             // FP32 loads the old q one plane ahead: two steps of mixed
             // 512x384x512 Crank-Nicolson (q only) 22.94 -> 22.77 ms, explicit
             // 256x192x256 2.36 -> 2.24, 384x256x384 6.11 -> 6.04.  It costs
@@ -1238,15 +1242,31 @@ template <typename T> struct FVImpl : FVBase {
         return DNS_OK;
     }
 
-    // z planes per block of the LDS z-march momentum kernel
-    int momentum_zc() const
+    // z planes per block of the LDS z-march momentum kernel (corr: its form
+    // that corrects u as it reads it): the march of 2 … 32 planes with the
+    // least rounds · (planes + 3), rounds of resident blocks (LDS and registers
+    // allow 3 per CU in FP64, 6 in FP32; corr 2 and 4) and 3 planes of prologue
+    // per block.  The longest march that fills one round (the rule before) is
+    // often 1.2 to 1.5 rounds: corr FP64, two steps of 256x192x256 3.71 ms at
+    // 32 planes, 3.55 at 16; 320x120x240 3.25 at 32, 2.94 at 8.  corr in FP32
+    // takes the shortest march within 10 %: its blocks overlap better than
+    // whole rounds and short marches share planes in L2 (512x384x512 15.30 at
+    // 32, 15.14 at 16).
+    int momentum_zc(bool corr = false) const
     {
-        const int nbx = ceil_div(g.nx, 64), nby = ceil_div(g.ny, 8);
-        const long round = 256L * (sizeof(T) == 8 ? 3 : 6);
-        int zc = 32;
-        while (zc > 2 && (long)nbx * nby * ceil_div(g.nz, zc) < round) zc /= 2;
-        if (const char *ez = getenv("DNS_MOM_ZC")) zc = std::max(1, atoi(ez)); // sweeps
-        return zc;
+        if (const char *ez = getenv("DNS_MOM_ZC")) return std::max(1, atoi(ez)); // sweeps
+        const long tiles = (long)ceil_div(g.nx, 64) * ceil_div(g.ny, 8);
+        const long slots = 256L * (sizeof(T) == 8 ? (corr ? 2 : 3) : corr ? 4 : 6);
+        auto cost = [&](int zc) { return ceil_div(tiles * ceil_div(g.nz, zc), slots) * (zc + 3); };
+        int best = 32;
+        for (int zc = 16; zc >= 2; zc /= 2)
+            if (cost(zc) < cost(best)) best = zc;
+        if (corr && sizeof(T) == 4) {
+            const long lim = cost(best);
+            for (int zc = best / 2; zc >= 4; zc /= 2)
+                if (10 * cost(zc) <= 11 * lim) best = zc;
+        }
+        return best;
     }
 
     // the kernel instances and launch shapes this handle's step uses
@@ -1269,11 +1289,13 @@ template <typename T> struct FVImpl : FVBase {
         else if (cn_tl && cn_seg) snprintf(cs, sizeof cs, "seg R=%d tl=%d thr=%d nl=%d", cn_seg, cn_tl, cn_nthr, cn_nl);
         else if (cn_tl) snprintf(cs, sizeof cs, "tile tl=%d thr=%d", cn_tl, cn_nthr);
         else snprintf(cs, sizeof cs, "sequential");
+        char stg[32] = "separate";
+        if (!plain && !imexy && stage_fused()) snprintf(stg, sizeof stg, "fused zc=%d", momentum_zc(true));
         const int n = snprintf(buf, (size_t)len,
                                "prec=%s; momentum=%s zc=%d; xpass=half %d %s; zpass=%s; "
-                               "ysolve=%s; cn=%s; pgrad=%s",
+                               "ysolve=%s; cn=%s; pgrad=%s; stages=%s",
                                plain ? "plain" : sizeof(T) == 8 ? "fp64" : "mixed", mom, momentum_zc(), g.nx / 2, xdesc,
-                               zs, ys, cs, pgrad_vec ? "vec" : "scalar");
+                               zs, ys, cs, pgrad_vec ? "vec" : "scalar", stg);
         if (n < 0 || n >= len) {
             set_error("describe: buffer of %d bytes too small", len);
             return DNS_EINVAL;
@@ -1339,14 +1361,29 @@ template <typename T> struct FVImpl : FVBase {
         return DNS_OK;
     }
 
+    // Explicit stages 2 and 3: the momentum kernel corrects u by −∇p as it reads
+    // it, so the pressure-gradient pass of stages 1 and 2 (7 of 31 fields a
+    // stage moves) is one read of p; the last stage keeps the pass, which
+    // stores u and its maxima.  Same operations on the same values: the
+    // results are bitwise the separate passes'.  Two steps of 512x384x512
+    // 31.4 -> 27.8 ms (mixed 16.8 -> 15.1), 256x192x256 3.96 -> 3.57, four of
+    // 128³ 1.43 -> 1.35 and 192x97x96 1.56 -> 1.47; but 128x96x96 1.10 -> 1.13
+    // and 96x65x80 (eight) 1.52 -> 1.57, where the two blocks per CU of ψ
+    // planes in LDS leave fewer loads in flight (mixed 96³ 0.84 -> 0.83).
+    bool stage_fused() const
+    {
+        return momentum_kind == 5 && g.nz >= 4 && N >= (sizeof(T) == 8 ? 3 << 19 : 3 << 18);
+    }
+
     int step_launch(double dt)
     {
         if (imexy) launch_cn_coeffs(dt);
         for (int s = 0; s < 3; ++s) {
             if (!imexy) {
-                DNS_TRY(launch_momentum(u, v, RK_A[s], dt, RK_B[s], true));
+                const bool fused = stage_fused();
+                DNS_TRY(launch_momentum(u, v, RK_A[s], dt, RK_B[s], true, s > 0 && fused ? p : nullptr));
                 DNS_TRY(launch_poisson(v, p, 0));
-                DNS_TRY(launch_pgrad(v, p, false, 0.0));
+                if (s == 2 || !fused) DNS_TRY(launch_pgrad(v, p, false, 0.0));
                 for (int c = 0; c < 3; ++c) std::swap(u[c], v[c]);
             } else {
                 DNS_TRY(launch_momentum(u, nullptr, RK_A[s], dt, 0.0, false));

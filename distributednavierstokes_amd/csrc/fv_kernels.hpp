@@ -85,6 +85,7 @@ template <typename T> struct MomentumArgs {
     T A, dt, nu, fx, fy, fz, epsy, B;
     T rdx, rdx2, rdz, rdz2;
     const double *dtp; // when set, Δt is read here (computed on the device) instead of dt
+    const T *psi;      // k_momentum_lz with CORR: u is corrected by −∇psi as it is read
 };
 
 // The three momentum components at one cell from its 27 stencil values
@@ -305,16 +306,18 @@ template <typename T> struct LZ {
     static constexpr int RP = 256 / LR;               // tile rows one pass of 256 threads covers
     static constexpr int NI = (NROW + RP - 1) / RP;   // vector items per thread per plane
     static constexpr int PL = NROW * P;               // one plane slot
+    static constexpr int PROW = SY + 1, PPL = PROW * P; // rows and slot of a ψ plane (CORR)
 };
 
-template <typename T, bool READ_Q, bool WRITE_V, bool QA = false>
-__global__ void __launch_bounds__(256) k_momentum_lz(MomentumArgs<T> a, FVGeom g, int zc)
+template <typename T, bool READ_Q, bool WRITE_V, bool QA = false, bool CORR = false>
+__global__ void __launch_bounds__(256, CORR ? 2 : 1) k_momentum_lz(MomentumArgs<T> a, FVGeom g, int zc)
 {
     resolve_dt(a);
     using L = LZ<T>;
     using VT = typename std::conditional<sizeof(T) == 8, double2, float4>::type;
     __shared__ __align__(16) T sm[3 * L::PL];
     __shared__ T met[6][L::TY];
+    __shared__ __align__(16) T sp[CORR ? 3 * L::PPL : 1]; // psi planes k' and k' + 1 of the u plane landing, and the next
     int bx, by, bz;
     xcd_block3(bx, by, bz);
     const int x0 = bx * L::TX, y0 = by * L::TY, k0 = bz * zc;
@@ -383,6 +386,86 @@ __global__ void __launch_bounds__(256) k_momentum_lz(MomentumArgs<T> a, FVGeom g
         hdst = r * L::P + (side ? L::V + w : L::V - 1);
         hsrc = fld[f];
     }
+    // CORR: an element of row js of component f becomes u − (ψ_B − ψ_A) m with
+    // ψ_A, ψ_B the two values of the gradient of k_pgrad at its own cell (LDS
+    // offsets within a plane of ψ; the z gradient takes ψ_B from plane k' + 1)
+    // and m its metric.  The ψ tile has rows y0 − 1 … y0 + TY + 1 (wrapped, or
+    // clamped at walls) and columns x0 − 1 … x0 + w + 1 (wrapped).
+    int pa[L::NI], pb[L::NI], pha = 0, phb = 0;
+    T pm[L::NI], phm = T(0);
+    bool pon[L::NI], phon = false, pz[L::NI], phz = false;
+    auto grad_at = [&](int f, int ly, int col, int &oa, int &ob, T &m, bool &zn, bool &on) {
+        const int j = y0 - 1 + ly;
+        int ra = ly; // tile row of ψ_A
+        if (f == 1 && g.wall && j == g.ny) ra = ly - 2;
+        int js;
+        T sg;
+        ghost(f, j, js, sg);
+        on = sg != T(0) && !(f == 1 && g.wall && js == g.ny - 1) && !(a.dtp && a.dt == T(0));
+        oa = ra * L::P + col;
+        ob = f == 0 ? oa + 1 : f == 1 ? oa + L::P : oa;
+        m = f == 0 ? a.rdx : f == 1 ? a.rdyu[js + 1] : a.rdz;
+        zn = f == 2;
+    };
+    if constexpr (CORR) {
+#pragma unroll
+        for (int s2 = 0; s2 < L::NI; ++s2) {
+            pa[s2] = pb[s2] = 0;
+            pm[s2] = T(0);
+            pon[s2] = pz[s2] = false;
+            const int r = r0 + s2 * L::RP;
+            if (r < L::NROW && vlane) grad_at(r / L::SY, r % L::SY, L::V + v * L::V, pa[s2], pb[s2], pm[s2], pz[s2], pon[s2]);
+        }
+        if (hlane) {
+            const int r = tid >> 1;
+            grad_at(r / L::SY, r % L::SY, (tid & 1) ? L::V + w : L::V - 1, pha, phb, phm, phz, phon);
+        }
+    }
+    // ψ tile loads: vector items and one halo value (columns −1, w, w + 1) per thread
+    constexpr int PNI = (L::PROW * L::LR + 255) / 256;
+    int psrc[PNI], pdst[PNI], phsrc = 0, phdst = -1;
+    if constexpr (CORR) {
+        auto prow = [&](int ly) {
+            const int j = y0 - 1 + ly;
+            if (g.wall) return j < 0 ? 0 : j >= g.ny ? g.ny - 1 : j;
+            return j < 0 ? j + g.ny : j >= g.ny ? (j - g.ny) % g.ny : j;
+        };
+#pragma unroll
+        for (int s2 = 0; s2 < PNI; ++s2) {
+            const int r = r0 + s2 * L::RP;
+            psrc[s2] = -1;
+            if (r < L::PROW && vlane) {
+                psrc[s2] = prow(r) * g.nx + x0 + v * L::V;
+                pdst[s2] = r * L::P + L::V + v * L::V;
+            }
+        }
+        if (tid < 3 * L::PROW) {
+            const int r = tid / 3, c = tid - 3 * r;
+            int i = c == 0 ? x0 - 1 : x0 + w + c - 1;
+            i = i < 0 ? i + g.nx : i >= g.nx ? i - g.nx : i;
+            phsrc = prow(r) * g.nx + i;
+            phdst = r * L::P + (c == 0 ? L::V - 1 : L::V + w + c - 1);
+        }
+    }
+    auto issue_p = [&](int k, VT (&vr)[PNI], T &hr) __attribute__((always_inline)) {
+        const int kw = k < 0 ? k + g.nz : (k >= g.nz ? k - g.nz : k);
+        const T *src = a.psi + plane * kw;
+#pragma unroll
+        for (int s2 = 0; s2 < PNI; ++s2)
+            if (psrc[s2] >= 0) vr[s2] = *reinterpret_cast<const VT *>(src + psrc[s2]);
+        if (phdst >= 0) hr = src[phsrc];
+    };
+    auto land_p = [&](int slot, VT (&vr)[PNI], T hr) __attribute__((always_inline)) {
+        T *dst = sp + slot * L::PPL;
+#pragma unroll
+        for (int s2 = 0; s2 < PNI; ++s2)
+            if (psrc[s2] >= 0) {
+                const VT x = vr[s2];
+                *reinterpret_cast<VT *>(dst + pdst[s2]) = x;
+            }
+        if (phdst >= 0) dst[phdst] = hr;
+    };
+
     // row metrics of the tile rows
     if (tid < L::TY) {
         const int j = min(y0 + tid, g.ny - 1), jj = j + 1;
@@ -396,8 +479,9 @@ __global__ void __launch_bounds__(256) k_momentum_lz(MomentumArgs<T> a, FVGeom g
 
     // two register sets alternate: while plane k is computed, planes k+2
     // (issued one plane earlier) and k+3 are in flight
-    VT vA[L::NI], vB[L::NI];
-    T hA = T(0), hB = T(0);
+    VT vA[L::NI], vB[L::NI], qA[PNI], qB[PNI];
+    T hA = T(0), hB = T(0), rA = T(0), rB = T(0);
+    int pslot = 0; // CORR: slot of the ψ plane of u plane k + 2
     auto issue = [&](int k, VT (&vr)[L::NI], T &hr) {
         const int kw = k < 0 ? k + g.nz : (k >= g.nz ? k - g.nz : k);
         const size_t pk = plane * kw;
@@ -406,19 +490,35 @@ __global__ void __launch_bounds__(256) k_momentum_lz(MomentumArgs<T> a, FVGeom g
             if (voff[s2] >= 0) vr[s2] = *reinterpret_cast<const VT *>(vsrc[s2] + pk + voff[s2]);
         if (hlane) hr = hsrc[pk + hoff];
     };
-    auto land = [&](int slot, VT (&vr)[L::NI], T hr) {
+    // (CORR: ψ of this plane in slot pk, of the next in slot pk + 1 mod 3)
+    auto land = [&](int slot, VT (&vr)[L::NI], T hr, int pk = 0) {
         T *dst = sm + slot * L::PL;
+        const T *p0 = sp + pk * L::PPL, *p1 = sp + (pk == 2 ? 0 : pk + 1) * L::PPL;
 #pragma unroll
         for (int s2 = 0; s2 < L::NI; ++s2) {
             if (voff[s2] >= 0) {
                 VT x = vr[s2];
                 T *e = reinterpret_cast<T *>(&x);
+                if constexpr (CORR) {
+                    const T *A = p0 + pa[s2], *B = (pz[s2] ? p1 : p0) + pb[s2];
+#pragma unroll
+                    for (int q = 0; q < L::V; ++q) {
+                        const T d = B[q] - A[q];
+                        e[q] = pon[s2] ? fma(-d, pm[s2], e[q]) : e[q];
+                    }
+                }
 #pragma unroll
                 for (int q = 0; q < L::V; ++q) e[q] = vsgn[s2] == T(0) ? T(0) : vsgn[s2] * e[q];
                 *reinterpret_cast<VT *>(dst + vdst[s2]) = x;
             }
         }
-        if (hlane) dst[hdst] = hsgn == T(0) ? T(0) : hsgn * hr;
+        if (hlane) {
+            if constexpr (CORR) {
+                const T d = (phz ? p1 : p0)[phb] - p0[pha];
+                hr = phon ? fma(-d, phm, hr) : hr;
+            }
+            dst[hdst] = hsgn == T(0) ? T(0) : hsgn * hr;
+        }
     };
 
     // old q of the plane being updated; QA: loaded one plane ahead
@@ -448,15 +548,39 @@ __global__ void __launch_bounds__(256) k_momentum_lz(MomentumArgs<T> a, FVGeom g
         issue(k0 + 1, vD, hD);
         if (QA) load_q(k0, qn);
         if (k0 + 1 < kend) issue(k0 + 2, vA, hA);
-        land(0, vB, hB);
-        land(1, vC, hC);
-        land(2, vD, hD);
+        if constexpr (CORR) {
+            // ψ up to plane kend + 1; plane k' sits in slot (k' − k0 + 1) mod 3
+            VT w0[PNI], w1[PNI], w2[PNI], w3[PNI], w4[PNI];
+            T g0 = T(0), g1 = T(0), g2 = T(0), g3 = T(0), g4 = T(0);
+            issue_p(k0 - 1, w0, g0);
+            issue_p(k0, w1, g1);
+            issue_p(k0 + 1, w2, g2);
+            issue_p(k0 + 2, w3, g3); // k0 + 2 <= kend + 1
+            if (k0 + 3 <= kend + 1) issue_p(k0 + 3, w4, g4);
+            if (k0 + 4 <= kend + 1) issue_p(k0 + 4, qA, rA);
+            land_p(0, w0, g0);
+            land_p(1, w1, g1);
+            land_p(2, w2, g2);
+            __syncthreads();
+            land(0, vB, hB, 0);
+            land(1, vC, hC, 1);
+            __syncthreads();
+            land_p(0, w3, g3);
+            if (k0 + 3 <= kend + 1) land_p(1, w4, g4);
+            __syncthreads();
+            land(2, vD, hD, 2);
+        } else {
+            land(0, vB, hB);
+            land(1, vC, hC);
+            land(2, vD, hD);
+        }
     }
     __syncthreads();
     int sM = 0, s0 = 1, sP = 2;
     // one plane: old q values, the loads of plane k+3, the update of plane k,
     // then plane k+2 (in cur) lands in the slot plane k−1 leaves
-    auto plane_step = [&](int k, VT (&cur)[L::NI], T &curh, VT (&nxt)[L::NI], T &nxth) {
+    auto plane_step = [&](int k, VT (&cur)[L::NI], T &curh, VT (&nxt)[L::NI], T &nxth, VT (&pcur)[PNI], T &pcurh,
+                          VT (&pnxt)[PNI], T &pnxth) {
         const int i = x0 + tx;
         T qo[2][3];
         if (!QA) load_q(k, qn);
@@ -466,6 +590,7 @@ __global__ void __launch_bounds__(256) k_momentum_lz(MomentumArgs<T> a, FVGeom g
             for (int c = 0; c < 3; ++c) qo[h][c] = qn[h][c];
         if (QA && k + 1 < kend) load_q(k + 1, qn);
         if (k + 2 < kend) issue(k + 3, nxt, nxth);
+        if (CORR && k + 5 <= kend + 1) issue_p(k + 5, pnxt, pnxth);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int ly = ty + 4 * h, j = y0 + ly;
@@ -485,7 +610,12 @@ __global__ void __launch_bounds__(256) k_momentum_lz(MomentumArgs<T> a, FVGeom g
         }
         __syncthreads(); // every wave is done with slot sM
         if (k + 1 < kend) {
-            land(sM, cur, curh);
+            land(sM, cur, curh, pslot);
+            if constexpr (CORR) {
+                // ψ of plane k + 4 replaces that of plane k + 1
+                if (k + 4 <= kend + 1) land_p(pslot == 0 ? 2 : pslot - 1, pcur, pcurh);
+                pslot = pslot == 2 ? 0 : pslot + 1;
+            }
             const int t = sM;
             sM = s0;
             s0 = sP;
@@ -494,8 +624,8 @@ __global__ void __launch_bounds__(256) k_momentum_lz(MomentumArgs<T> a, FVGeom g
         __syncthreads();
     };
     for (int k = k0; k < kend; k += 2) {
-        plane_step(k, vA, hA, vB, hB);
-        if (k + 1 < kend) plane_step(k + 1, vB, hB, vA, hA);
+        plane_step(k, vA, hA, vB, hB, qA, rA, qB, rB);
+        if (k + 1 < kend) plane_step(k + 1, vB, hB, vA, hA, qB, rB, qA, rA);
     }
 }
 
