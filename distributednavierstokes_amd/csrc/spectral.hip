@@ -470,6 +470,9 @@ template <typename T> struct SpecImpl : SpecBase {
         if (MODE == XMID_RHS && xr_wave)
             hipLaunchKernelGGL((k_sp_xrhs256<T>), dim3(ceil_div((long)g.n * g.n, 4)), dim3(SP_NTHR),
                                (size_t)(TW4S_LEN + 257 + 4 * 256) * sizeof(cplx<T>), st, a, g);
+        else if (MODE == XMID_VMAX && xr_wave)
+            hipLaunchKernelGGL((k_sp_xrhs256<T, true>), dim3(ceil_div((long)g.n * g.n, 4)), dim3(SP_NTHR),
+                               (size_t)(TW4S_LEN + 257 + 4 * 256) * sizeof(cplx<T>), st, a, g);
         else if (MODE == XMID_RHS && xr_lpi)
             hipLaunchKernelGGL((k_sp_xrhs<T, SP_XEPT>), dim3(xr_blocks), dim3(SP_NTHR), ldsxr, st, a, g, fdh, xr_lpi);
         else
@@ -755,7 +758,8 @@ template <typename T> struct SpecImpl : SpecBase {
     {
         DNS_TRY(backward_yz());
         DNS_TRY(xpass<XMID_VMAX>(red));
-        return vmax_final(x2_lpw ? x2_blocks : ceil_div((long)g.n * g.n, lpb), out);
+        const int nparts = x2_lpw ? x2_blocks : xr_wave ? rhs_parts() : ceil_div((long)g.n * g.n, lpb);
+        return vmax_final(nparts, out);
     }
 
     long cube_count(int r) const

@@ -1014,7 +1014,8 @@ __device__ __forceinline__ void wave_fft256(cplx<T> (&a)[4], cplx<T> *sh, const 
 // instead of 8·8·4).  No workgroup barrier after the twiddle staging.  One
 // vmax partial per block.  LDS: the transform twiddles (stage_tw4s, 272), the
 // 257 real-transform twiddles, 4 × 256 complex.
-template <typename T>
+// VMAX: only the velocity bound (512³ FP64 1.76 ms in k_sp_xmid, 0.58 here).
+template <typename T, bool VMAX = false>
 __global__ void __launch_bounds__(256) k_sp_xrhs256(XMidArgs<T> a, SpecGeom g)
 {
     constexpr int N = 256;
@@ -1081,7 +1082,7 @@ __global__ void __launch_bounds__(256) k_sp_xrhs256(XMidArgs<T> a, SpecGeom g)
     for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
     if (lane == 0) red[wv] = mx;
 #pragma unroll
-    for (int p = 0; p < 6; ++p) {
+    for (int p = 0; p < (VMAX ? 0 : 6); ++p) {
         const int ca = p < 3 ? p : (p == 3 ? 0 : p == 4 ? 1 : 2);
         const int cb = p < 3 ? p : (p == 3 ? 1 : p == 4 ? 2 : 0);
         cplx<T> z[4];
