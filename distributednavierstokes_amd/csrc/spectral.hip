@@ -95,14 +95,14 @@ template <typename T> struct SpecImpl : SpecBase {
     int x2_lpw = 0, x2_waves = 0, x2_blocks = 0; // wavefront x pass (k_sp_x2): lines per wavefront (0: not used), launch
     size_t ldsxr = 0;
     size_t lds = 0, ldss = 0, ldsx = 0;
-    double *red = nullptr, *redout = nullptr, *factors = nullptr, *pinned = nullptr;
+    double *red = nullptr, *factors = nullptr, *pinned = nullptr;
     size_t redcap = 0;
 
     ~SpecImpl() override
     {
         if (st) hipStreamSynchronize(st);
         timer.flush();
-        void *ptrs[] = {uh, ustart, du, P, Q, phys, twN, twx, twn, red, redout, factors, aux, tphys};
+        void *ptrs[] = {uh, ustart, du, P, Q, phys, twN, twx, twn, red, factors, aux, tphys};
         for (void *p_ : ptrs)
             if (p_) hipFree(p_);
         if (pinned) hipHostFree(pinned);
@@ -221,7 +221,6 @@ template <typename T> struct SpecImpl : SpecBase {
         }
         redcap = std::max<size_t>({(size_t)SP_REDB * 4, 2 * ((size_t)g.n * g.n / lpb + 16), 2 * ((size_t)x2_blocks + 64)}); // (64: a partly filled block per slab)
         DNS_TRY(dalloc(&red, redcap));
-        DNS_TRY(dalloc(&redout, 64));
         DNS_TRY(dalloc(&factors, 4096));
         DNS_HIP_CHECK(hipHostMalloc((void **)&pinned, sizeof(double) * 4096));
         return DNS_OK;
@@ -725,12 +724,18 @@ template <typename T> struct SpecImpl : SpecBase {
 
     int vmax_final(int nparts, double *out)
     {
-        // two levels: up to 256 blocks into the scratch half of red, then one
-        const int G = std::min(256, std::max(1, nparts / 1024));
-        hipLaunchKernelGGL(k_max_mid, dim3(G), dim3(SP_NTHR), 0, st, red, nparts, 1, red + redcap / 2);
-        hipLaunchKernelGGL(k_max_final, dim3(1), dim3(SP_NTHR), 0, st, red + redcap / 2, G, 1, redout);
+        // two levels: up to 256 blocks into the scratch half of red, then one;
+        // up to 4096 partials in one.  The result goes straight to the pinned
+        // host buffer (a copy of 8 bytes costs a launch of its own)
+        const double *part = red;
+        if (nparts > 4096) {
+            const int G = std::min(256, nparts / 1024);
+            hipLaunchKernelGGL(k_max_mid, dim3(G), dim3(SP_NTHR), 0, st, red, nparts, 1, red + redcap / 2);
+            part = red + redcap / 2;
+            nparts = G;
+        }
+        hipLaunchKernelGGL(k_max_final, dim3(1), dim3(SP_NTHR), 0, st, part, nparts, 1, pinned);
         DNS_HIP_CHECK(hipGetLastError());
-        DNS_HIP_CHECK(hipMemcpyAsync(pinned, redout, sizeof(double), hipMemcpyDeviceToHost, st));
         DNS_HIP_CHECK(hipStreamSynchronize(st));
         *out = pinned[0];
         return DNS_OK;
@@ -796,10 +801,9 @@ template <typename T> struct SpecImpl : SpecBase {
             hipLaunchKernelGGL((k_sp_shells<T>), dim3(nb), dim3(SP_NTHR),
                                sizeof(double) * nsh + (sizeof(double) + sizeof(int)) * SP_NTHR, st, uh, s0, nsh, r,
                                count, g, red);
-        hipLaunchKernelGGL(k_bins_final, dim3(ceil_div(nsh, SP_NTHR)), dim3(SP_NTHR), 0, st, red, nb, nsh, factors);
+        hipLaunchKernelGGL(k_bins_final, dim3(ceil_div(nsh, SP_NTHR)), dim3(SP_NTHR), 0, st, red, nb, nsh, pinned);
         timer.end(SFAM_FORCE);
         DNS_HIP_CHECK(hipGetLastError());
-        DNS_HIP_CHECK(hipMemcpyAsync(pinned, factors, sizeof(double) * nsh, hipMemcpyDeviceToHost, st));
         DNS_HIP_CHECK(hipStreamSynchronize(st));
         for (int q = 0; q < nsh; ++q) E[q] = pinned[q];
         return DNS_OK;
@@ -811,16 +815,25 @@ template <typename T> struct SpecImpl : SpecBase {
             set_error("invalid shell range");
             return DNS_EINVAL;
         }
-        for (int q = 0; q < nsh; ++q) pinned[q] = f[q];
-        DNS_HIP_CHECK(hipMemcpyAsync(factors, pinned, sizeof(double) * nsh, hipMemcpyHostToDevice, st));
+        // a few factors (forcing) travel as kernel arguments: no copy, and no
+        // wait for the pinned buffer they would be staged in
+        ShellFactors few{};
+        const bool args = nsh <= SHELL_ARGS;
+        if (args) {
+            for (int q = 0; q < nsh; ++q) few.f[q] = f[q];
+        } else {
+            for (int q = 0; q < nsh; ++q) pinned[q] = f[q];
+            DNS_HIP_CHECK(hipMemcpyAsync(factors, pinned, sizeof(double) * nsh, hipMemcpyHostToDevice, st));
+        }
         int r = s0 + nsh - 1;
         long count = cube_count(r);
         int nb = (int)std::max<long>(1, std::min<long>(SP_REDB, (count + SP_NTHR - 1) / SP_NTHR));
         timer.begin(SFAM_FORCE);
-        hipLaunchKernelGGL((k_sp_rescale<T>), dim3(nb), dim3(SP_NTHR), 0, st, uh, s0, nsh, r, count, factors, g);
+        hipLaunchKernelGGL((k_sp_rescale<T>), dim3(nb), dim3(SP_NTHR), 0, st, uh, s0, nsh, r, count,
+                           args ? nullptr : factors, few, g);
         timer.end(SFAM_FORCE);
         DNS_HIP_CHECK(hipGetLastError());
-        DNS_HIP_CHECK(hipStreamSynchronize(st)); // the pinned staging buffer is reused
+        if (!args) DNS_HIP_CHECK(hipStreamSynchronize(st)); // the pinned staging buffer is reused
         return DNS_OK;
     }
 
@@ -838,9 +851,8 @@ template <typename T> struct SpecImpl : SpecBase {
     {
         int nb = (int)std::min<long>(SP_REDB, ceil_div((long)ns, SP_NTHR));
         hipLaunchKernelGGL((k_sp_energy<T>), dim3(nb), dim3(SP_NTHR), 0, st, uh, g, reinterpret_cast<dd *>(red));
-        hipLaunchKernelGGL(k_dd_final, dim3(2), dim3(SP_NTHR), 0, st, reinterpret_cast<dd *>(red), nb, 2, redout);
+        hipLaunchKernelGGL(k_dd_final, dim3(2), dim3(SP_NTHR), 0, st, reinterpret_cast<dd *>(red), nb, 2, pinned);
         DNS_HIP_CHECK(hipGetLastError());
-        DNS_HIP_CHECK(hipMemcpyAsync(pinned, redout, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
         DNS_HIP_CHECK(hipStreamSynchronize(st));
         if (e) *e = pinned[0];
         if (diss) *diss = visc * pinned[1];

@@ -769,17 +769,28 @@ __global__ void __launch_bounds__(256) k_sp_shells_w(const cplx<T> *uh, int s0, 
         part[(size_t)blockIdx.x * ns + b] = ((bins[b] + bins[ns + b]) + bins[2 * ns + b]) + bins[3 * ns + b];
 }
 
+// factors of up to SHELL_ARGS shells as a kernel argument (factors == null)
+constexpr int SHELL_ARGS = 16;
+struct ShellFactors {
+    double f[SHELL_ARGS];
+};
+
 template <typename T>
 __global__ void __launch_bounds__(256) k_sp_rescale(cplx<T> *uh, int s0, int ns, int r, long count,
-                                                    const double *factors, SpecGeom g)
+                                                    const double *factors, ShellFactors few, SpecGeom g)
 {
+    __shared__ double sf[SHELL_ARGS];
+#pragma unroll
+    for (int q = 0; q < SHELL_ARGS; ++q)
+        if (threadIdx.x == q) sf[q] = few.f[q];
+    __syncthreads();
     const size_t cs = (size_t)g.K * g.m * g.m;
     for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < count; t += (long)gridDim.x * blockDim.x) {
         int i, j, k;
         sp_cube(t, r, g, i, j, k);
         int sh = sp_shell(i, j, k, g) - s0;
         if (sh < 0 || sh >= ns) continue;
-        T f = T(factors[sh]);
+        T f = T(factors ? factors[sh] : sf[sh]);
         size_t base = i + (size_t)g.K * (j + (size_t)g.m * k);
         for (int c = 0; c < 3; ++c) uh[base + c * cs] = cscale<T>(uh[base + c * cs], f);
     }
