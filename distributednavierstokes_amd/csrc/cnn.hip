@@ -267,8 +267,11 @@ struct CNN {
         const dim3 grd((unsigned)ceil_div((long)M * M, 256), (unsigned)M, (unsigned)(Vn / Vs)), blk(256);
         const size_t lds = conv_plane_lds(M, np, ca.kin);
         constexpr int NB = EPI == 1 ? 1 : 2; // 6 outputs, else 64
-        if (ca.kin == 64) hipLaunchKernelGGL((k_conv_plane<MC, NB, 64, EPI>), grd, blk, lds, s, ca, geom(Vn));
-        else hipLaunchKernelGGL((k_conv_plane<MC, NB, 16, EPI>), grd, blk, lds, s, ca, geom(Vn));
+        if (ca.kin == 64) {
+            hipLaunchKernelGGL((k_conv_plane<MC, NB, 64, EPI>), grd, blk, lds, s, ca, geom(Vn));
+        } else if constexpr (EPI != 1) {
+            hipLaunchKernelGGL((k_conv_plane<MC, NB, 16, EPI>), grd, blk, lds, s, ca, geom(Vn));
+        }
     }
     // The output convolution where no backward pass follows: k_conv_out sums
     // dx last, so its results differ from k_conv_plane's in the last FP32 bits,
@@ -301,7 +304,7 @@ struct CNN {
         // and k_conv16 (other M), ms per two training steps: 16 × 64³
         // 16.7 / 32.0, 4 × 48³ 2.45 / 6.30, 4 × 32³ 1.00 / 1.69; five LES
         // steps of 36³ 2.40 / 5.86, 80³ 10.3 / 23.7.
-        if (conv_pf && conv_wlds && Vn / Vs <= 65535 && (ca.kin == 16 || ca.kin == 64) && np == (EPI == 1 ? 32 : 64) &&
+        if (conv_pf && conv_wlds && Vn / Vs <= 65535 && (ca.kin == 64 || (ca.kin == 16 && EPI != 1)) && np == (EPI == 1 ? 32 : 64) &&
             conv_plane_lds(M, np, ca.kin) <= max_lds) {
             if (M == 64) conv_plane<64, EPI>(ca, np, Vn, s);
             else if (M == 32) conv_plane<32, EPI>(ca, np, Vn, s);

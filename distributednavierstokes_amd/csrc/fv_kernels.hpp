@@ -297,6 +297,11 @@ __global__ void __launch_bounds__(256) k_momentum_slab(MomentumArgs<T> a, FVGeom
 // earlier.  Rows outside the wall follow the ldc/ldf ghost rules.
 // Grid (ceil(nx/64), ceil(ny/8), ceil(nz/zc)) of 256 threads, XCD-ordered;
 // LDS 3 planes × 3 components × 10 rows × (64 + 2V) + metric rows.
+// CORR: u is read uncorrected and becomes u − ∇ψ as a plane lands, with the
+// operations of k_pgrad; ψ planes k+2 … k+4 wait in a ring of three (18 KB in
+// FP64, so two blocks per CU instead of three).  Bound by HBM: 256x192x256
+// FP64 287 µs for 13 fields (1374 MB of counter traffic, 4.8 TB/s), where the
+// form without and the pass it replaces took 253 + 115 µs.
 template <typename T> struct LZ {
     static constexpr int TX = 64, TY = 8, SY = TY + 2;
     static constexpr int V = 16 / sizeof(T);          // elements per 16-byte load
