@@ -276,15 +276,15 @@ struct CNN {
     // The output convolution where no backward pass follows: k_conv_out sums
     // dx last, so its results differ from k_conv_plane's in the last FP32 bits,
     // and a gradient would see them where a BF16 dy rounds the other way.
-    bool conv_out(const ConvArgs &ca, long Vn, hipStream_t s)
+    bool conv_out(const ConvArgs &ca, const StressOut &so, long Vn, hipStream_t s)
     {
         const size_t lds = M <= 256 ? conv_out_lds(M, ca.nout) : 0;
         if (!conv_pf || mfma_k8 || ca.kin != 64 || ca.nout > CO_NMAX || M > 256 || Vn / Vs > 65535 || lds > max_lds) return false;
         const dim3 grd((unsigned)ceil_div(M, conv_out_rows(M)), (unsigned)M, (unsigned)(Vn / Vs));
-        if (M == 64) hipLaunchKernelGGL((k_conv_out<64>), grd, dim3(256), lds, s, ca, geom(Vn));
-        else if (M == 32) hipLaunchKernelGGL((k_conv_out<32>), grd, dim3(256), lds, s, ca, geom(Vn));
-        else if (M == 16) hipLaunchKernelGGL((k_conv_out<16>), grd, dim3(256), lds, s, ca, geom(Vn));
-        else hipLaunchKernelGGL((k_conv_out<0>), grd, dim3(256), lds, s, ca, geom(Vn));
+        if (M == 64) hipLaunchKernelGGL((k_conv_out<64>), grd, dim3(256), lds, s, ca, so, geom(Vn));
+        else if (M == 32) hipLaunchKernelGGL((k_conv_out<32>), grd, dim3(256), lds, s, ca, so, geom(Vn));
+        else if (M == 16) hipLaunchKernelGGL((k_conv_out<16>), grd, dim3(256), lds, s, ca, so, geom(Vn));
+        else hipLaunchKernelGGL((k_conv_out<0>), grd, dim3(256), lds, s, ca, so, geom(Vn));
         return true;
     }
     template <int EPI> void conv(const ConvArgs &ca, int np, long Vn, hipStream_t s)
@@ -342,9 +342,10 @@ struct CNN {
     }
 
     // forward of the first nb batch slots of x0; the FP32 output lands in y
-    // (nb M³ × 6); the layers' z (half of the bytes a hidden layer writes)
+    // (nb M³ × 6), or as so (one sample) asks: cleared where y was written
+    // after all; the layers' z (half of the bytes a hidden layer writes)
     // only where a backward pass follows (keep_z)
-    int forward(hipStream_t s, int nb, bool keep_z = false)
+    int forward(hipStream_t s, int nb, bool keep_z = false, StressOut *so = nullptr)
     {
         const long Vn = (long)nb * Vs;
         for (int l = 0; l < 4; ++l) {
@@ -365,7 +366,10 @@ struct CNN {
             } else {
                 ca.yout = y;
                 ca.ldo = 6;
-                if (keep_z || !conv_out(ca, Vn, s)) conv<1>(ca, c.np, Vn, s);
+                if (keep_z || !conv_out(ca, so ? *so : StressOut{}, Vn, s)) {
+                    conv<1>(ca, c.np, Vn, s);
+                    if (so) *so = StressOut{};
+                }
             }
         }
         DNS_HIP_CHECK(hipGetLastError());
@@ -692,8 +696,12 @@ struct CNN {
         DNS_HIP_CHECK(hipEventRecord(ev_in, st));
         DNS_HIP_CHECK(hipStreamWaitEvent(s, ev_in, 0));
         hipLaunchKernelGGL((k_velocity_to_bf16<T>), dim3(ceil_div(Vs, 256)), dim3(256), 0, s, vel, Vs, (float)(1.0 / su), x0);
-        DNS_TRY(forward(s, 1));
-        hipLaunchKernelGGL((k_stress_to_planar<T>), dim3(ceil_div(Vs, 256)), dim3(256), 0, s, y, Vs, stau, tau);
+        StressOut so{nullptr, nullptr, stau};
+        if constexpr (sizeof(T) == 4) so.f = tau;
+        else so.d = tau;
+        DNS_TRY(forward(s, 1, false, &so));
+        if (!so.f && !so.d)
+            hipLaunchKernelGGL((k_stress_to_planar<T>), dim3(ceil_div(Vs, 256)), dim3(256), 0, s, y, Vs, stau, tau);
         DNS_HIP_CHECK(hipGetLastError());
         DNS_HIP_CHECK(hipEventRecord(ev_out, s));
         DNS_HIP_CHECK(hipStreamWaitEvent(st, ev_out, 0));

@@ -4,7 +4,9 @@ voxel-tile kernels that serve any grid."""
 import numpy as np
 import pytest
 
+import distributednavierstokes_amd as dns
 from distributednavierstokes_amd.cnn import SFSNet
+from distributednavierstokes_amd.spectral import DeviceState
 from oracle import oracle_cnn as oc
 
 pytestmark = pytest.mark.gpu
@@ -39,3 +41,27 @@ def test_against_voxel_tiles(M, B, monkeypatch):
         for m in (27 * co * ci, co):
             assert np.linalg.norm(g[off:off + m] - gr[off:off + m]) <= 2e-5 * np.linalg.norm(gr[off:off + m])
             off += m
+
+
+# planar FP32 and FP64 stress from the output convolution, whole rows of a block and not
+@pytest.mark.parametrize("n", [16, 24, 30, 64])
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+def test_les_increment_against_voxel_tiles(n, T, monkeypatch):
+    """The change of an LES step with the stress written by the output
+    convolution or by a pass over its result: to the bound of the network's
+    BF16 inputs (3e-2, as against the FP64 restatement), since the velocity of
+    the later stages passes through that rounding."""
+    inc = []
+    for kind in (None, "direct"):
+        if kind:
+            monkeypatch.setenv("DNS_CNN_CONV", kind)
+        s = dns.spectral_setup(n=n, visc=1e-2, T=T)
+        dns.spectral_randomfield_(DeviceState(s), s, totalenergy=1.0, kpeak=2, seed=3)
+        net = SFSNet(M=n, batch=1, seed=0)
+        net.set_params((np.random.default_rng(n).standard_normal(net.nparams) * 0.08).astype(np.float32))
+        before = np.array(s.download())
+        dns.spectral_solve_(uh=DeviceState(s), setup=s, tlims=(0.0, 1e-3), dt=1e-3, closure=net)
+        inc.append(np.array(s.download()) - before)
+    err = np.linalg.norm(inc[0] - inc[1]) / np.linalg.norm(inc[1])
+    print(f"LES increment n={n} {T.__name__}: {err:.2e}", flush=True)
+    assert err <= 3e-2
