@@ -614,11 +614,33 @@ template <typename T> struct SpecImpl : SpecBase {
         return DNS_OK;
     }
 
-    cplx<T> *aux = nullptr; // τ of the SFS recipe (K, m, m, 6), LES handles only
+    cplx<T> *aux = nullptr; // τ̂ of the last SFS sample or closure step (K, m, m, 6), LES handles only
+    bool aux_from_tphys = false; // a closure step left its stress in tphys only
     int ensure_aux()
     {
         if (!aux) DNS_TRY(dalloc(&aux, 6 * ns));
         return DNS_OK;
+    }
+
+    // τ̂ for a reader: the stress of a closure step is transformed when it is
+    // asked for (the step itself adds it to the products in physical space)
+    int sfs_stress()
+    {
+        if (aux_from_tphys) {
+            DNS_TRY(ensure_aux());
+            DNS_TRY(stress_to_aux());
+            aux_from_tphys = false;
+        }
+        if (!aux) {
+            set_error("no SFS sample on this handle");
+            return DNS_EINVAL;
+        }
+        return DNS_OK;
+    }
+    int stress_to_aux()
+    {
+        DNS_TRY(phys_to_spec_into(tphys, aux));
+        return phys_to_spec_into(tphys + (size_t)3 * g.n * g.n * g.n, aux + 3 * ns);
     }
 
     int phys_to_spec() override
@@ -658,6 +680,7 @@ template <typename T> struct SpecImpl : SpecBase {
                 DNS_TRY(backward_yz());
                 DNS_TRY(xpass<XMID_C2R>(nullptr));
                 DNS_TRY(cnn_stress<T>(net, phys, tphys, g.n, st));
+                aux_from_tphys = true;
                 DNS_TRY(xpass<XMID_RHS>(s == 0 ? red : nullptr, nullptr, tphys));
                 DNS_TRY(zfwd(6));
                 DNS_TRY(ystage<0>(s, dt));
@@ -671,8 +694,7 @@ template <typename T> struct SpecImpl : SpecBase {
             DNS_TRY(backward_yz());
             DNS_TRY(xpass<XMID_C2R>(red + redcap / 2));
             DNS_TRY(cnn_stress<T>(net, phys, tphys, g.n, st));
-            DNS_TRY(phys_to_spec_into(tphys, aux));
-            DNS_TRY(phys_to_spec_into(tphys + 3 * n3, aux + 3 * ns));
+            DNS_TRY(stress_to_aux());
             DNS_TRY(backward_yz());
             DNS_TRY(xpass<XMID_RHS>(s == 0 ? red : red + redcap / 2));
             DNS_TRY(zfwd(6));
@@ -685,10 +707,7 @@ template <typename T> struct SpecImpl : SpecBase {
     // Appends the physical (ū, τ) of the last SFS sample to the network's dataset.
     int append_sample(dns_cnn *net)
     {
-        if (!aux) {
-            set_error("no SFS sample on this handle");
-            return DNS_EINVAL;
-        }
+        DNS_TRY(sfs_stress());
         DNS_TRY(ensure_phys());
         const size_t n3 = (size_t)g.n * g.n * g.n;
         if (!tphys) DNS_TRY(dalloc(&tphys, 6 * n3));
@@ -885,6 +904,7 @@ int sfs_sample(SpecImpl<T> *D, SpecImpl<T> *L, double delta_fac, int protectshel
     DNS_TRY(D->products());
     DNS_HIP_CHECK(hipStreamSynchronize(D->st));
     DNS_TRY(L->ensure_aux());
+    L->aux_from_tphys = false;
     const double M = L->g.n;
     const double delta = delta_fac * L->l / M;
     const double kb = L->g.kfac * (protectshells + 1);
@@ -903,10 +923,7 @@ template <typename T> int sfs_get(SpecImpl<T> *L, double *ubar, double *tau)
 {
     if (ubar) DNS_TRY(L->get_state(ubar, 0));
     if (tau) {
-        if (!L->aux) {
-            set_error("no SFS sample on this handle");
-            return DNS_EINVAL;
-        }
+        DNS_TRY(L->sfs_stress());
         const size_t n6 = 6 * L->ns;
         std::vector<cplx<T>> b(n6);
         DNS_HIP_CHECK(hipMemcpyAsync(b.data(), L->aux, sizeof(cplx<T>) * n6, hipMemcpyDeviceToHost, L->st));
@@ -922,10 +939,7 @@ template <typename T> int sfs_get(SpecImpl<T> *L, double *ubar, double *tau)
 // Physical ū (M³×3) and τ (M³×6) of the last sample, host copies.
 template <typename T> int sfs_physical(SpecImpl<T> *L, double *ubar, double *tau)
 {
-    if (!L->aux) {
-        set_error("no SFS sample on this handle");
-        return DNS_EINVAL;
-    }
+    DNS_TRY(L->sfs_stress());
     const size_t n3 = (size_t)L->g.n * L->g.n * L->g.n;
     std::vector<T> b(3 * n3);
     auto fetch = [&](double *dst) -> int {

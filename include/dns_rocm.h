@@ -254,7 +254,10 @@ int dns_spec_load(dns_spec *h, const char *prefix, double *time, int64_t *step);
  * T⅔ keeps), the same l and precision, and M/2 <= the DNS kcut.  The results
  * stay on `les`: its state holds ū, its SFS buffer holds τ̂ (6 components). */
 int dns_sfs_sample(dns_spec *dns, dns_spec *les, double delta_fac, int32_t protectshells);
-/* Copies ū (K, m, m, 3) and τ̂ (K, m, m, 6) of the LES handle (either may be NULL). */
+/* Copies ū (K, m, m, 3) and τ̂ (K, m, m, 6) of the LES handle (either may be
+ * NULL): τ̂ of its last dns_sfs_sample, or of the last stage of its last
+ * dns_les_closure_step when that is newer (dns_sfs_physical and dns_sfs_append
+ * likewise; the first such read after a step is a pipeline call). */
 int dns_sfs_get(dns_spec *les, double *ubar_hat, double *tau_hat);
 /* Physical ū (M, M, M, 3) and τ (M, M, M, 6) on the LES grid (host). */
 int dns_sfs_physical(dns_spec *les, double *ubar, double *tau);
