@@ -273,18 +273,20 @@ struct CNN {
             hipLaunchKernelGGL((k_conv_plane<MC, NB, 16, EPI>), grd, blk, lds, s, ca, geom(Vn));
         }
     }
-    // The output convolution where no backward pass follows: k_conv_out sums
-    // dx last, so its results differ from k_conv_plane's in the last FP32 bits,
-    // and a gradient would see them where a BF16 dy rounds the other way.
-    bool conv_out(const ConvArgs &ca, const StressOut &so, long Vn, hipStream_t s)
+    // The output convolution of the LES stress: k_conv_out sums dx last, so its
+    // results differ from k_conv_plane's in the last FP32 bits.  A gradient
+    // would see them where a BF16 dy rounds the other way, and forward, eval and
+    // predict give the values the training loss is made of: those keep the
+    // plane kernel (36 against 26 µs for one 64³ sample).
+    bool conv_out(const ConvArgs &ca, const StressOut &so, hipStream_t s)
     {
         const size_t lds = M <= 256 ? conv_out_lds(M, ca.nout) : 0;
-        if (!conv_pf || mfma_k8 || ca.kin != 64 || ca.nout > CO_NMAX || M > 256 || Vn / Vs > 65535 || lds > max_lds) return false;
-        const dim3 grd((unsigned)ceil_div(M, conv_out_rows(M)), (unsigned)M, (unsigned)(Vn / Vs));
-        if (M == 64) hipLaunchKernelGGL((k_conv_out<64>), grd, dim3(256), lds, s, ca, so, geom(Vn));
-        else if (M == 32) hipLaunchKernelGGL((k_conv_out<32>), grd, dim3(256), lds, s, ca, so, geom(Vn));
-        else if (M == 16) hipLaunchKernelGGL((k_conv_out<16>), grd, dim3(256), lds, s, ca, so, geom(Vn));
-        else hipLaunchKernelGGL((k_conv_out<0>), grd, dim3(256), lds, s, ca, so, geom(Vn));
+        if (!conv_pf || mfma_k8 || ca.kin != 64 || ca.nout > CO_NMAX || M > 256 || lds > max_lds) return false;
+        const dim3 grd((unsigned)ceil_div(M, conv_out_rows(M)), (unsigned)M);
+        if (M == 64) hipLaunchKernelGGL((k_conv_out<64>), grd, dim3(256), lds, s, ca, so, geom(Vs));
+        else if (M == 32) hipLaunchKernelGGL((k_conv_out<32>), grd, dim3(256), lds, s, ca, so, geom(Vs));
+        else if (M == 16) hipLaunchKernelGGL((k_conv_out<16>), grd, dim3(256), lds, s, ca, so, geom(Vs));
+        else hipLaunchKernelGGL((k_conv_out<0>), grd, dim3(256), lds, s, ca, so, geom(Vs));
         return true;
     }
     template <int EPI> void conv(const ConvArgs &ca, int np, long Vn, hipStream_t s)
@@ -342,9 +344,9 @@ struct CNN {
     }
 
     // forward of the first nb batch slots of x0; the FP32 output lands in y
-    // (nb M³ × 6), or as so (one sample) asks: cleared where y was written
-    // after all; the layers' z (half of the bytes a hidden layer writes)
-    // only where a backward pass follows (keep_z)
+    // (nb M³ × 6), or planar and scaled as so (one sample) asks: cleared where
+    // y was written after all; the layers' z (half of the bytes a hidden layer
+    // writes) only where a backward pass follows (keep_z)
     int forward(hipStream_t s, int nb, bool keep_z = false, StressOut *so = nullptr)
     {
         const long Vn = (long)nb * Vs;
@@ -366,7 +368,7 @@ struct CNN {
             } else {
                 ca.yout = y;
                 ca.ldo = 6;
-                if (keep_z || !conv_out(ca, so ? *so : StressOut{}, Vn, s)) {
+                if (!so || !conv_out(ca, *so, s)) {
                     conv<1>(ca, c.np, Vn, s);
                     if (so) *so = StressOut{};
                 }

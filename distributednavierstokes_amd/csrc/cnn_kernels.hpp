@@ -790,7 +790,7 @@ __global__ void __launch_bounds__(256) k_conv_plane(ConvArgs a, ConvGeom g)
     }
 }
 
-// Output convolution (64 → nout channels, 3 nout <= 32, FP32 result): the three
+// Output convolution of the LES stress (64 → nout channels, 3 nout <= 32): the three
 // dx taps are columns of one product, P[v][(dx, n)] = Σ_{dz, dy, k}
 // W[dx, dy, dz][n][k] in[v + (0, dy, dz)][k], and out[v][n] = b[n] +
 // Σ_dx P[v + dx][(dx, n)] is formed from LDS at the end.  So 9 taps of a
@@ -800,7 +800,7 @@ __global__ void __launch_bounds__(256) k_conv_plane(ConvArgs a, ConvGeom g)
 // A block takes R = min(256 / M, M) whole rows of one (z, b) plane, four
 // wavefronts of two 32-voxel tiles; rows ylo − 1 … ylo + R and the weights of
 // one dz are staged at a time (MC = M: the next ones in flight meanwhile).
-// Grid (ceil(M / R), M, B); M <= 256.  LDS: conv_out_lds.
+// Grid (ceil(M / R), M); M <= 256.  LDS: conv_out_lds.
 constexpr int CO_KS = 72, CO_PITCH = 33, CO_NMAX = 10; // halves per voxel / weight row, floats per voxel of P, most outputs
 inline int conv_out_rows(int M) { return std::min(256 / M, M); }
 inline size_t conv_out_lds(int M, int nout)
@@ -808,9 +808,8 @@ inline size_t conv_out_lds(int M, int nout)
     return std::max((size_t)((conv_out_rows(M) + 2) * M + 9 * nout) * 2 * CO_KS, (size_t)256 * CO_PITCH * sizeof(float));
 }
 
-// so: the LES stress instead of yout: planar (nout, M³), scale · result, in FP32
-// or FP64 (one sample; a pass of its own took 4.7 µs per stage at 64³, five LES
-// steps 3.83 -> 3.70 ms).
+// The result: planar (nout, M³), scale · result, in FP32 or FP64 (one sample; a
+// pass of its own took 4.7 µs per stage at 64³, five LES steps 3.83 -> 3.70 ms).
 struct StressOut {
     float *f;
     double *d;
@@ -823,7 +822,7 @@ template <int MC> __global__ void __launch_bounds__(256) k_conv_out(ConvArgs a, 
     constexpr int MB = 2, KS = CO_KS;
     const int M = MC ? MC : g.M, R = min(256 / M, M);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, row = lane & 31, h = lane >> 5;
-    const int ylo = blockIdx.x * R, nr = min(R, M - ylo), z = blockIdx.y, b = blockIdx.z, nout = a.nout, nj = 3 * nout;
+    const int ylo = blockIdx.x * R, nr = min(R, M - ylo), z = blockIdx.y, nout = a.nout, nj = 3 * nout;
     unsigned short *sa = reinterpret_cast<unsigned short *>(smem_raw), *sw = sa + (R + 2) * M * KS;
     f32x16 acc[MB];
 #pragma unroll
@@ -842,8 +841,7 @@ template <int MC> __global__ void __launch_bounds__(256) k_conv_out(ConvArgs a, 
         int ys = ylo - 1 + rr, zs = z + dzi - 1;
         ys = ys < 0 ? ys + M : ys >= M ? ys - M : ys;
         zs = zs < 0 ? zs + M : zs >= M ? zs - M : zs;
-        return *reinterpret_cast<const u32x4 *>(gin + ((size_t)x + (size_t)M * (ys + (size_t)M * (zs + (size_t)M * b))) * 64 +
-                                                8 * c8);
+        return *reinterpret_cast<const u32x4 *>(gin + ((size_t)x + (size_t)M * (ys + (size_t)M * zs)) * 64 + 8 * c8);
     };
     auto place = [&](int e, u32x4 v) __attribute__((always_inline)) {
         *reinterpret_cast<u32x4 *>(sa + (e >> 3) * KS + 8 * (e & 7)) = v;
@@ -905,17 +903,15 @@ template <int MC> __global__ void __launch_bounds__(256) k_conv_out(ConvArgs a, 
             if (j < nj) P[(64 * wave + 32 * mb + row) * CO_PITCH + j] = acc[mb][r];
         }
     __syncthreads();
-    const size_t v0 = (size_t)M * (ylo + (size_t)M * (z + (size_t)M * b));
-    const bool planar = so.f || so.d;
+    const size_t v0 = (size_t)M * (ylo + (size_t)M * z);
     const int nv = nr * M;
     const size_t vs = (size_t)M * M * M;
     for (int e = tid; e < nv * nout; e += 256) {
-        const int v = planar ? e % nv : e / nout, n = planar ? e / nv : e - v * nout, x = v % M;
+        const int n = e / nv, v = e - n * nv, x = v % M;
         const int vm = x == 0 ? v + M - 1 : v - 1, vp = x == M - 1 ? v - (M - 1) : v + 1;
         const float r = (P[vm * CO_PITCH + n] + P[v * CO_PITCH + nout + n] + P[vp * CO_PITCH + 2 * nout + n]) + a.bias[n];
         if (so.f) so.f[n * vs + v0 + v] = (float)(so.scale * (double)r);
-        else if (so.d) so.d[n * vs + v0 + v] = so.scale * (double)r;
-        else a.yout[(v0 + v) * a.ldo + n] = r;
+        else so.d[n * vs + v0 + v] = so.scale * (double)r;
     }
 }
 
