@@ -151,6 +151,7 @@ template <typename T> struct FVImpl : FVBase {
     bool pgrad_vec = false; // k_pgrad_vec (16-byte accesses) instead of k_pgrad
     bool xwave = false;     // x passes by wavefront lane groups (nx/2 in 16..256, a power of two)
     bool umax_valid = false; // upart holds max |u_c| partials of the current u
+    bool fuse_stages = true; // DNS_FV_STAGES (stage_fused)
     int momentum_kind = 5; // 5 LDS z-march (k_momentum_lz), 3 slab-ordered (k_momentum_slab), 1 direct (k_momentum)
     // reference-structured ("plain") step: extra arrays, allocated on first use
     bool plain = false;
@@ -219,6 +220,8 @@ template <typename T> struct FVImpl : FVBase {
                                                    : 5;
             // the LDS z-march loads whole rows as 16-byte vectors
             if (momentum_kind == 5 && nx % (16 / (int)sizeof(T)) != 0) momentum_kind = 3;
+            const char *es = getenv("DNS_FV_STAGES");
+            fuse_stages = !(es && !strcmp(es, "separate"));
         }
         visc = P->visc;
         for (int c = 0; c < 3; ++c) f[c] = P->bodyforce[c];
@@ -1370,9 +1373,10 @@ template <typename T> struct FVImpl : FVBase {
     // 128³ 1.43 -> 1.35 and 192x97x96 1.56 -> 1.47; but 128x96x96 1.10 -> 1.13
     // and 96x65x80 (eight) 1.52 -> 1.57, where the two blocks per CU of ψ
     // planes in LDS leave fewer loads in flight (mixed 96³ 0.84 -> 0.83).
+    // DNS_FV_STAGES=separate keeps the passes.
     bool stage_fused() const
     {
-        return momentum_kind == 5 && g.nz >= 4 && N >= (sizeof(T) == 8 ? 3 << 19 : 3 << 18);
+        return fuse_stages && momentum_kind == 5 && g.nz >= 4 && N >= (sizeof(T) == 8 ? 3 << 19 : 3 << 18);
     }
 
     int step_launch(double dt)
