@@ -692,25 +692,16 @@ template <typename T> struct FVImpl : FVBase {
             const int zc = momentum_zc(psi != nullptr);
             dim3 grd(nbx, nby, ceil_div(g.nz, zc));
             if (psi) {
-                hipLaunchKernelGGL((k_momentum_lz<T, true, true, sizeof(T) == 4, true>), grd, dim3(256), 0, st, a, g, zc);
+                hipLaunchKernelGGL((k_momentum_lz<T, true, true, true>), grd, dim3(256), 0, st, a, g, zc);
                 timer.end(FAM_MOM);
                 DNS_HIP_CHECK(hipGetLastError());
                 return DNS_OK;
             }
-            // FP32 loads the old q one plane ahead: two steps of mixed
-            // 512x384x512 Crank-Nicolson (q only) 22.94 -> 22.77 ms, explicit
-            // 256x192x256 2.36 -> 2.24, 384x256x384 6.11 -> 6.04.  It costs
-            // one of five wavefronts per SIMD: explicit 512x384x512 (u' written
-            // as well) 16.85 -> 16.99, so not there; FP64 would keep two of
-            // three wavefronts and gains nothing.
             if (write_v) {
-                constexpr bool F32 = sizeof(T) == 4;
-                if (rq && F32 && N <= (64 << 20))
-                    hipLaunchKernelGGL((k_momentum_lz<T, true, true, F32>), grd, dim3(256), 0, st, a, g, zc);
-                else if (rq) hipLaunchKernelGGL((k_momentum_lz<T, true, true>), grd, dim3(256), 0, st, a, g, zc);
+                if (rq) hipLaunchKernelGGL((k_momentum_lz<T, true, true>), grd, dim3(256), 0, st, a, g, zc);
                 else hipLaunchKernelGGL((k_momentum_lz<T, false, true>), grd, dim3(256), 0, st, a, g, zc);
             } else {
-                if (rq) hipLaunchKernelGGL((k_momentum_lz<T, true, false, sizeof(T) == 4>), grd, dim3(256), 0, st, a, g, zc);
+                if (rq) hipLaunchKernelGGL((k_momentum_lz<T, true, false>), grd, dim3(256), 0, st, a, g, zc);
                 else hipLaunchKernelGGL((k_momentum_lz<T, false, false>), grd, dim3(256), 0, st, a, g, zc);
             }
             timer.end(FAM_MOM);

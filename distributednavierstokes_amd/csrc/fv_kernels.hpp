@@ -293,8 +293,7 @@ __global__ void __launch_bounds__(256) k_momentum_slab(MomentumArgs<T> a, FVGeom
 // are fixed for the whole march, so a plane costs a few adds per load.  The
 // loads of plane k+3 are issued before plane k is computed, and plane k+2
 // (issued one plane earlier) lands in LDS after it: two planes in flight per
-// thread.  The old q values are read before the plane loads, with QA one plane
-// earlier.  Rows outside the wall follow the ldc/ldf ghost rules.
+// thread.  The old q values are read before the plane loads.  Rows outside the wall follow the ldc/ldf ghost rules.
 // Grid (ceil(nx/64), ceil(ny/8), ceil(nz/zc)) of 256 threads, XCD-ordered;
 // LDS 3 planes × 3 components × 10 rows × (64 + 2V) + metric rows.
 // CORR: u is read uncorrected and becomes u − ∇ψ as a plane lands, with the
@@ -314,7 +313,7 @@ template <typename T> struct LZ {
     static constexpr int PROW = SY + 1, PPL = PROW * P; // rows and slot of a ψ plane (CORR)
 };
 
-template <typename T, bool READ_Q, bool WRITE_V, bool QA = false, bool CORR = false>
+template <typename T, bool READ_Q, bool WRITE_V, bool CORR = false>
 __global__ void __launch_bounds__(256, CORR ? 2 : 1) k_momentum_lz(MomentumArgs<T> a, FVGeom g, int zc)
 {
     resolve_dt(a);
@@ -526,7 +525,14 @@ __global__ void __launch_bounds__(256, CORR ? 2 : 1) k_momentum_lz(MomentumArgs<
         }
     };
 
-    // old q of the plane being updated; QA: loaded one plane ahead
+    // Old q of the plane being updated; QA: loaded one plane ahead.  Only the
+    // FP32 form that corrects u (its psi planes set the occupancy) gains by it,
+    // ms per step against loading it first: 256x192x256 0.963 / 0.953,
+    // 384x256x384 3.04 / 3.01, 512x384x512 7.26 / 7.27.  Without CORR it costs
+    // a fifth of the wavefronts: Crank-Nicolson 256³ 1.984 / 1.972 but
+    // 384x201x240 2.319 / 2.338 and 512x384x512 11.20 / 11.21, explicit
+    // 96x65x80 0.2247 / 0.2256.
+    constexpr bool QA = CORR && sizeof(T) == 4;
     const int tx = tid & 63, ty = __builtin_amdgcn_readfirstlane(tid >> 6);
     T qn[2][3];
     auto load_q = [&](int k, T (&qd)[2][3]) {
