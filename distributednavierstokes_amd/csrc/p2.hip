@@ -26,9 +26,8 @@ bool p2_launch(P2Kind kind, const P2Args<double> &a, dim3 grid, hipStream_t st)
 
 template <typename T> bool p2_serves(P2Kind kind, int n)
 {
-    if (kind == P2_STAGE && n > p2_stage_max<T>()) return false;
 #define X(A, B) \
-    if (n == (A) * (B)) return true;
+    if (n == (A) * (B)) return kind != P2_STAGE || p2_stage_shape(A, B);
     P2_SHAPES_0
     P2_SHAPES_1
     P2_SHAPES_2

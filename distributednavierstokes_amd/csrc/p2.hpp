@@ -37,12 +37,15 @@ template <typename T> struct P2Args {
     double dscale;
 };
 
-// Longest line of P2_STAGE.  Beyond it three accumulators per retained
-// output and the transform's points fill the registers at one wavefront per
-// SIMD, and the block kernel k_sp_ystage is faster (forced box, ms per step:
-// 256³ FP64 3.07 against 3.14, 288³ FP64 4.52 against 4.25, 512³ FP64 21.3
-// against 20.3; 384³ FP32 5.14-5.19 against 5.22, 480³ FP32 10.1 against 9.9).
-template <typename T> constexpr int p2_stage_max() { return sizeof(T) == 8 ? 256 : 400; }
+// Line lengths N1·N2 of P2_STAGE.  Three accumulators per retained output and
+// the transform's points fill the registers of longer lines at one wavefront
+// per SIMD; a first radix up to 16 holds on longest.  Elsewhere the block
+// kernel k_sp_ystage serves (µs per launch of this kernel / of that one, forced
+// box on MI355X: FP64 180 90 / 120, 192 120 / 126, 240 213 / 252, 256 229 / 253,
+// but 200 193 / 135, 216 247 / 205, 250 345 / 264; FP32 180 32 / 56, 192 51-56 /
+// 55, 240 96 / 130, 256 125 / 130, but 200 90 / 66, 250 152 / 137, 288 251 / 207,
+// 320 287 / 263, 360 412 / 397, and 324, 384 and 400 equal).
+constexpr bool p2_stage_shape(int n1, int n2) { return n1 * n2 <= 180 || (n1 <= 16 && n1 * n2 <= 256); }
 
 // False when no kernel serves (T, n, kind): the caller takes the LDS tiles.
 bool p2_launch(P2Kind kind, const P2Args<float> &a, dim3 grid, hipStream_t st);

@@ -316,7 +316,7 @@ template <typename T, int N1, int N2> inline bool p2_go(int kind, const P2Args<T
         case P2_BACK: hipLaunchKernelGGL((k_p2_back<T, N1, N2>), grid, blk, lds, st, a); return true;
         case P2_FWD: hipLaunchKernelGGL((k_p2_fwd<T, N1, N2>), grid, blk, lds, st, a); return true;
         case P2_STAGE:
-            if constexpr (F::N <= p2_stage_max<T>()) {
+            if constexpr (p2_stage_shape(N1, N2)) {
                 hipLaunchKernelGGL((k_p2_stage<T, N1, N2>), grid, blk, lds, st, a);
                 return true;
             }
