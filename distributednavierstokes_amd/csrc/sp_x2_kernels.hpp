@@ -3,6 +3,7 @@
 
 #include "fft_reg.hpp"
 #include "sp_x2.hpp"
+#include "sp_x2_shapes.hpp"
 
 namespace dns {
 
@@ -182,10 +183,13 @@ __global__ void __launch_bounds__(256, 2) k_sp_x2(X2Args<T> a)
 
 template <typename T, int N1, int N2> inline bool sp_x2_go(const X2Args<T> &a, int blocks, int waves, hipStream_t st)
 {
-    constexpr int LS = N1 * (N2 | 1), LPW = 64 / N1;
-    const size_t lds = sizeof(cplx<T>) * (size_t)(LS + N1 * N2 + waves * LPW * LS);
-    hipLaunchKernelGGL((k_sp_x2<T, N1, N2>), dim3(blocks), dim3(64 * waves), lds, st, a);
-    return true;
+    if constexpr (sp_x2_shape<T>(N2)) {
+        constexpr int LS = N1 * (N2 | 1), LPW = 64 / N1;
+        const size_t lds = sizeof(cplx<T>) * (size_t)(LS + N1 * N2 + waves * LPW * LS);
+        hipLaunchKernelGGL((k_sp_x2<T, N1, N2>), dim3(blocks), dim3(64 * waves), lds, st, a);
+        return true;
+    }
+    return false;
 }
 
 }  // namespace dns

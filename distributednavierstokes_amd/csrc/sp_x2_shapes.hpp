@@ -4,6 +4,12 @@
 // with the block kernels.  X(N1, N2); two lists, one per compilation unit.
 #pragma once
 
+namespace dns {
+// FP64 stops at N2 = 12: the registers of three components of 15 or 16 points
+// per lane spill (450-540 B per lane).
+template <typename T> constexpr bool sp_x2_shape(int n2) { return sizeof(T) == 4 || n2 <= 12; }
+}  // namespace dns
+
 #define SP_X2_SHAPES_LO \
     X(4, 4) \
     X(6, 3) \

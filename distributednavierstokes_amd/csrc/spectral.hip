@@ -26,8 +26,7 @@ static const double W_DC[3] = {8.0 / 15.0, 2.0 / 15.0, 1.0 / 3.0};
 constexpr int SP_XEPT = 8, SP_SEPT = 8, SP_MAXO = 6, SP_NTHR = 256, SP_REDB = 1024;
 
 // The wavefront x pass (sp_x2.hpp): lines per wavefront of half length N
-// (0: not served) and its launch.  FP64 stops at N2 = 12: the registers of
-// three components of 15 or 16 points per lane spill (450-540 B per lane).
+// (0: not served) and its launch.
 bool sp_x2_f32_lo(const X2Args<float> &, int, int, hipStream_t);
 bool sp_x2_f32_hi(const X2Args<float> &, int, int, hipStream_t);
 bool sp_x2_f64_lo(const X2Args<double> &, int, int, hipStream_t);
@@ -43,7 +42,7 @@ static bool sp_x2_go(const X2Args<double> &a, int blocks, int waves, hipStream_t
 template <typename T> static int sp_x2_lines(int N)
 {
 #define X(A, B) \
-    if (N == (A) * (B) && (sizeof(T) == 4 || (B) <= 12)) return 64 / (A);
+    if (N == (A) * (B)) return sp_x2_shape<T>(B) ? 64 / (A) : 0;
     SP_X2_SHAPES_LO
     SP_X2_SHAPES_HI
 #undef X
