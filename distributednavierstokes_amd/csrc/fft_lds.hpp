@@ -444,9 +444,17 @@ __device__ __forceinline__ void fft_lds_groups(cplx<T> *buf, int nlines, int ls,
     __syncthreads();
 }
 
+// fft_lds over sub-batches of at most sub lines (tw[t] = exp(-2πi t / n)).
+template <typename T, int EPT, bool INV, int NT = 0>
+__device__ __forceinline__ void fft_lds_lines(cplx<T> *buf, int nlines, int ls, const FFTDesc &d, const cplx<T> *tw, int sub)
+{
+    for (int sb = 0; sb < nlines; sb += sub)
+        fft_lds<T, EPT, INV, NT>(buf + (size_t)sb * ls, min(sub, nlines - sb), ls, d, tw);
+}
+
 // The batched LDS transforms of a tile: lane groups for the lengths they
-// serve (16 ... 512, powers of two, nlines a multiple of the lines per
-// wavefront), otherwise fft_lds over sub-batches of at most sub lines.
+// serve (64 ... 512, powers of two, nlines a multiple of the lines per
+// wavefront), otherwise fft_lds_lines.
 // Whether fft_lds_tile transforms nlines lines of n points by lane groups.
 __device__ inline bool fft_tile_groups(int n, int nlines)
 {
@@ -478,8 +486,7 @@ __device__ __forceinline__ void fft_lds_tile(cplx<T> *buf, int nlines, int ls, c
     if (n == 256) return fft_lds_groups<T, INV, 256, NT, PTW>(buf, nlines, ls, tw);
     if (n == 128 && nlines % 2 == 0) return fft_lds_groups<T, INV, 128, NT, PTW>(buf, nlines, ls, tw);
     if (n == 64 && nlines % 4 == 0) return fft_lds_groups<T, INV, 64, NT, PTW>(buf, nlines, ls, tw);
-    for (int sb = 0; sb < nlines; sb += sub)
-        fft_lds<T, EPT, INV, NT>(buf + (size_t)sb * ls, min(sub, nlines - sb), ls, d, tw);
+    fft_lds_lines<T, EPT, INV, NT>(buf, nlines, ls, d, tw, sub);
 }
 
 // Line tiles in HBM: a block holds tb lines (line b valid for b < nb) of n

@@ -151,13 +151,13 @@ __global__ void __launch_bounds__(NT, 2) k_sp_yback(const cplx<T> *uh, cplx<T> *
     extern __shared__ unsigned char smem_raw[];
     cplx<T> *buf = reinterpret_cast<cplx<T> *>(smem_raw);
     const int n = g.n, ls = sp_line_stride<T>(n), K = g.K, m = g.m;
-    const cplx<T> *twl = stage_tile_twiddles<T>(buf + (size_t)tb * ls, tw, n, tb);
+    const cplx<T> *twl = stage_twiddles<T>(buf + (size_t)tb * ls, tw, n);
     int bxr, byr, bzr;
     xcd_block3(bxr, byr, bzr);
     const int i0 = bxr * tb, kz = byr, c = bzr, nb = min(tb, K - i0);
     pencil_load_compact<T, EPT, NT>(buf, ls, uh + i0 + (size_t)K * m * (kz + (size_t)m * c), K, nb, tb, ftb, g);
     __syncthreads();
-    fft_lds_tile<T, EPT, true, 0, true>(buf, tb, ls, d, twl, tbf);
+    fft_lds_lines<T, EPT, true>(buf, tb, ls, d, twl, tbf);
     tile_store<T, EPT, NT>(buf, ls, B1 + i0 + (size_t)K * n * (kz + (size_t)m * c), K, nb, tb, ftb, n);
 }
 
@@ -170,13 +170,13 @@ __global__ void __launch_bounds__(NT, 2) k_sp_zback(const cplx<T> *B1, cplx<T> *
     extern __shared__ unsigned char smem_raw[];
     cplx<T> *buf = reinterpret_cast<cplx<T> *>(smem_raw);
     const int n = g.n, ls = sp_line_stride<T>(n), K = g.K, m = g.m;
-    const cplx<T> *twl = stage_tile_twiddles<T>(buf + (size_t)tb * ls, tw, n, tb);
+    const cplx<T> *twl = stage_twiddles<T>(buf + (size_t)tb * ls, tw, n);
     int bxr, byr, bzr;
     xcd_block3(bxr, byr, bzr);
     const int i0 = bxr * tb, y = byr, c = bzr, nb = min(tb, K - i0);
     pencil_load_compact<T, EPT, NT>(buf, ls, B1 + i0 + (size_t)K * (y + (size_t)n * m * c), K * n, nb, tb, ftb, g);
     __syncthreads();
-    fft_lds_tile<T, EPT, true, 0, true>(buf, tb, ls, d, twl, tbf);
+    fft_lds_lines<T, EPT, true>(buf, tb, ls, d, twl, tbf);
     tile_store<T, EPT, NT>(buf, ls, P + i0 + (size_t)K * (y + (size_t)n * n * c), K * n, nb, tb, ftb, n);
 }
 
@@ -189,13 +189,13 @@ __global__ void __launch_bounds__(NT, 2) k_sp_zfwd(const cplx<T> *P, cplx<T> *Q,
     extern __shared__ unsigned char smem_raw[];
     cplx<T> *buf = reinterpret_cast<cplx<T> *>(smem_raw);
     const int n = g.n, ls = sp_line_stride<T>(n), K = g.K, m = g.m;
-    const cplx<T> *twl = stage_tile_twiddles<T>(buf + (size_t)tb * ls, tw, n, tb);
+    const cplx<T> *twl = stage_twiddles<T>(buf + (size_t)tb * ls, tw, n);
     int bxr, byr, bzr;
     xcd_block3(bxr, byr, bzr);
     const int i0 = bxr * tb, y = byr, p = bzr, nb = min(tb, K - i0);
     tile_load<T, EPT, NT, SP_LOAD_U(EPT)>(buf, ls, P + i0 + (size_t)K * (y + (size_t)n * n * p), K * n, nb, tb, ftb, n);
     __syncthreads();
-    fft_lds_tile<T, EPT, false, 0, true>(buf, tb, ls, d, twl, tbf);
+    fft_lds_lines<T, EPT, false>(buf, tb, ls, d, twl, tbf);
     pencil_store_fine<T, EPT, NT, false>(buf, ls, Q + i0 + (size_t)K * (y + (size_t)n * m * p), K * n, nb, tb, ftb, g,
                                          T(1));
 }
@@ -210,13 +210,13 @@ __global__ void __launch_bounds__(NT, 2) k_sp_yfwd(const cplx<T> *Q, cplx<T> *ou
     extern __shared__ unsigned char smem_raw[];
     cplx<T> *buf = reinterpret_cast<cplx<T> *>(smem_raw);
     const int n = g.n, ls = sp_line_stride<T>(n), K = g.K, m = g.m;
-    const cplx<T> *twl = stage_tile_twiddles<T>(buf + (size_t)tb * ls, tw, n, tb);
+    const cplx<T> *twl = stage_twiddles<T>(buf + (size_t)tb * ls, tw, n);
     int bxr, byr, bzr;
     xcd_block3(bxr, byr, bzr);
     const int i0 = bxr * tb, kc = byr, p = bzr, nb = min(tb, K - i0);
     tile_load<T, EPT, NT, SP_LOAD_U(EPT)>(buf, ls, Q + i0 + (size_t)K * n * (kc + (size_t)m * p), K, nb, tb, ftb, n);
     __syncthreads();
-    fft_lds_tile<T, EPT, false, 0, true>(buf, tb, ls, d, twl, tbf);
+    fft_lds_lines<T, EPT, false>(buf, tb, ls, d, twl, tbf);
     const T inv = T(1.0 / ((double)n * n * n));
     pencil_store_fine<T, EPT, NT, true>(buf, ls, out + i0 + (size_t)K * m * (kc + (size_t)m * p), K, nb, tb, ftb, g, inv);
 }
