@@ -205,13 +205,12 @@ template <typename T> struct SpecImpl : SpecBase {
             // 128-byte rows; measured against the LDS tiles on the forced box,
             // ms per step: 96³ FP64 0.45 -> 0.31, 192³ FP64 1.49 -> 1.32, 512³
             // FP64 21.6 -> 20.3; 96³ FP32 0.41 -> 0.26, 384³ FP32 5.88 -> 5.16,
-            // 512³ FP32 11.7 -> 11.0 (64-byte rows 12-15 % slower there)
+            // 512³ FP32 11.7 -> 11.0.  64-byte rows in FP32, twice the blocks:
+            // 12-15 % slower there, 2-9 % from 100 to 160 points and below 48,
+            // and within 1.5 % either way between (48 ... 96).
             p2_pencil = p2_serves<T>(P2_FWD, g.n);
             p2_stage = p2_serves<T>(P2_STAGE, g.n);
-            // (small FP32 boxes: 64-byte rows make twice the blocks, two forced
-            // steps of 48³ 0.355 -> 0.330 ms, 64³ 0.405 -> 0.375, 128³ 0.582 ->
-            // 0.573; 192³ 1.219 -> 1.242, and five LES steps of 32³ 1.88 -> 1.92)
-            p2_lb = sizeof(T) == 8 || (g.n >= 40 && g.n <= 128) ? 3 : 4;
+            p2_lb = sizeof(T) == 8 ? 3 : 4;
             // 64-row slabs of P where they fit the memory-side cache and the
             // whole of P does not (ms per step: 384³ FP32 5.20 -> 4.89, 256³
             // FP64 3.06 -> 2.84; 32 rows 5.22 and 3.00).  Longer lines would
