@@ -362,8 +362,13 @@ template <typename T> struct SpecImpl : SpecBase {
         DNS_TRY(yback(uh));
         const size_t K = g.K, n = g.n, m = g.m;
         int part = 0;
-        for (int y0 = 0; y0 < g.n; y0 += slab_y) {
-            const int ys = std::min(slab_y, g.n - y0);
+        for (int y0 = 0, ys; y0 < g.n; y0 += ys) {
+            // up to three quarters of a slab more join the last one: launches of
+            // few rows cost more than they keep in the cache (ms per step with
+            // a slab of their own, joined, and no slabs: 216³ FP64 1.809 / 1.752 /
+            // 1.791, 270³ FP32 1.874 / 1.800 / 1.759, 300³ FP32 2.328 / 2.267 /
+            // 2.374)
+            ys = g.n - y0 <= slab_y + 3 * slab_y / 4 ? g.n - y0 : slab_y;
             P2Args<T> a = p2_args();
             a.src = Q + K * y0;
             a.sstride = (int)(K * n);
