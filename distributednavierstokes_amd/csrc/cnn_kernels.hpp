@@ -8,9 +8,10 @@
 // for the forward pass, and the transposed copy WT[o][k][n] for the data
 // gradient.  FP32 master weights and Adam moments live beside them.
 //
-// MFMA: v_mfma_f32_32x32x8_bf16 (wave64): C[32×32] += A[32×8]·B[8×32]; lane l
-// supplies A[l%32][4(l/32)..4(l/32)+3] and B[4(l/32)..+3][l%32]; it receives
-// C[8(r/4) + 4(l/32) + r%4][l%32] in accumulator r = 0..15.
+// MFMA: v_mfma_f32_32x32x16_bf16 (wave64): C[32×32] += A[32×16]·B[16×32]; lane l
+// supplies A[l%32][8(l/32)..+7] and B[8(l/32)..+7][l%32]; it receives
+// C[8(r/4) + 4(l/32) + r%4][l%32] in accumulator r = 0..15.  (The voxel-tile
+// kernels k_conv and k_conv_wgrad take v_mfma_f32_32x32x8_bf16: 4 values a lane.)
 #pragma once
 
 #include "common.hpp"

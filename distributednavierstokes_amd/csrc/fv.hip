@@ -1364,6 +1364,10 @@ template <typename T> struct FVImpl : FVBase {
     // 128³ 1.43 -> 1.35 and 192x97x96 1.56 -> 1.47; but 128x96x96 1.10 -> 1.13
     // and 96x65x80 (eight) 1.52 -> 1.57, where the two blocks per CU of ψ
     // planes in LDS leave fewer loads in flight (mixed 96³ 0.84 -> 0.83).
+    // Between 1.6 and 2.4 M cells FP64 grids whose tiles the correcting form
+    // marches in twice as many planes per block lose by it (eight steps of
+    // 96x140x128 3.02 -> 3.25, 200x97x90 3.06 -> 3.35, 96x256x96 3.46 -> 3.57;
+    // 128x120x108 2.50 -> 2.45, 144³ 4.51 -> 4.21).
     // DNS_FV_STAGES=separate keeps the passes.
     bool stage_fused() const
     {

@@ -1320,8 +1320,8 @@ __global__ void __launch_bounds__(256, 2) k_thomas_seg(cplx<T> *__restrict__ A, 
 // Once t >= tend − 1e-10(|tend| + 1) (the end test of solve!,
 // src/timestep.jl:102) it writes Δt = 0 and neither advances t nor counts a
 // step: the step that follows leaves u unchanged (q = 0, u′ = u, and the
-// pressure-gradient pass skips on Δt = 0).  One block of 1024 threads: the
-// last reduction level and Δt in one launch (as launches of their own, two
+// pressure-gradient pass skips on Δt = 0).  One block (256 threads for up to
+// 256 partials, else 1024): the last reduction level and Δt in one launch (as launches of their own, two
 // reduction levels and Δt took 15 µs of a 200 µs step of 96x65x80, so 6.4).
 __global__ void __launch_bounds__(1024) k_cfl_dt(const double *part, int nparts, double dx, double dymin, double dz,
                                                  double diff, double cfl, double tend, double *t, double *dt,

@@ -8,7 +8,7 @@ configurations run:
   segments of 24 rows, 256-point half-length x lines, 512-point z lines
   (the FP32 16-line z tile);
 - HIT 512³, kcut 170 (C4): one IF-RK3 step of the production pipeline, and
-  the same step at 128³ and 256³ (their lane-group pencil FFT lengths).
+  the same step at 128³ and 256³ (two-step pencil and x lines).
 
 The FV cases are thin slabs that keep one production dimension each, so the
 FP64 oracle finishes in seconds; `dns_fv_describe` shows that a slab runs the
@@ -159,8 +159,8 @@ def test_hit_step_matches_band_limited_oracle(n, precision):
     the 2/3 cut kcut = n/3 on a field with |k_i| <= 2, against the oracle's
     step of the same modes at n = 48, kcut = 16 (no truncation or aliasing
     differs between the two).  n = 512 is the production pipeline (the
-    four-step 256-point x lines, the 512-point lane-group pencils); 128 and
-    256 run the 128- and 256-point lane-group pencil FFTs."""
+    four-step 256-point x lines, the 512-point two-step pencils); 128 and 256
+    run two-step pencils, x lines and IF stages."""
     visc, dt = 0.01, 0.02
     small = OracleSpectral(SpectralProblem(n=48, kcut=16, visc=visc))
     uh = small.velocityfield(lambda x, y, z: np.sin(x + 2 * y) * np.cos(z) + 0.4 * np.cos(2 * z - y),

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 # the smallest length, lengths of the first radices 5 ... 16 (the larger ones run in
-# test_gpu_fv_p2.py and the 512³ step), K below one tile, kcut far below n/3
+# test_gpu_spectral_shapes.py and the 512³ step), K below one tile, kcut far below n/3
 @pytest.mark.parametrize("n,kcut", [(24, 8), (30, 10), (36, 3), (50, 16), (64, 21), (80, 26), (90, 30), (108, 36), (128, 20),
                                     (150, 50)])
 @pytest.mark.parametrize("T", [np.float64, np.float32])
@@ -51,7 +51,7 @@ def test_p2_transforms_rhs_step_products(n, kcut, T):
 
 def test_slab_step_216():
     """A grid whose product pencils exceed the memory-side cache takes the z
-    and x passes in 64-row slabs (here 64, 64, 64 and 24): step and max Σ|v|
+    and x passes in 64-row slabs (here 64, 64 and 88 rows): step and max Σ|v|
     against the oracle."""
     n = 216
     s = dns.spectral_setup(n=n, visc=5e-3)

@@ -81,7 +81,7 @@ def device(a):
 
 # x lines: n = 2·12·8 ... 2·16·16, FP64 up to N2 = 12 (the others by the block kernels); pencils: every even
 # length of the lists from 162 on; the IF stage by either kernel; 64-row slabs in FP32 from 256 on, the last one
-# ragged at 270 ... 432; kcut at n / 3 and well below it
+# ragged at 270 ... 360; kcut at n / 3 and well below it
 FP32 = [162, 180, 192, 200, 216, 240, 250, 256, 270, 288, 300, 320, 324, 360, 384, 400, 432, 450, 480, 486, 500]
 FP64 = [180, 192, 200, 240, 256, 270, 288, 300, 320, 384, 432]
 

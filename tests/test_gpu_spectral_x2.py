@@ -9,8 +9,8 @@ from oracle.oracle import OracleSpectral
 
 pytestmark = pytest.mark.gpu
 
-# smallest and largest half lengths, every radix of the small DFTs (2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16), odd and
-# prime-power half lengths, line counts that leave partly filled wavefronts
+# half lengths 16 ... 80 (from the smallest on): splits with the radices 3, 4, 5, 6, 8, 9, 10 and 15, odd and prime-power
+# half lengths, line counts that leave partly filled wavefronts; the longer ones run in test_gpu_spectral_shapes.py
 SIZES = [32, 36, 40, 50, 54, 64, 72, 96, 120, 150, 160]
 
 
